@@ -375,3 +375,43 @@ def test_gather_i64_segments(dev, target):
     torch.cuda.synchronize()
     got = vals.tolist() if target == "mapped" else dst.tolist()
     assert got[: len(want)] == want and got[len(want):] == [-7] * 8
+
+
+@pytest.mark.parametrize("ps,seqs", [(16, [1]), (64, [5000]), (1, [3, 700]), (16, [257, 256, 255, 1, 4097]),
+                                     (7, [20] * 600), (64, [63, 64, 65] * 30)])
+def test_alloc_extend_many_tokens_per_request(dev, ps, seqs):
+    """Requests of more tokens than one workgroup, or one round of them, takes (256 and 4096), more requests than
+    the grid is wide (512), and page remainders, against the oracle allocator; every other request starts inside
+    a page, and request 0 appends nothing when there is a second one."""
+    lib = _lib()
+    rng = np.random.default_rng(len(seqs) + ps)
+    pre = [int(rng.integers(1, 3 * ps + 1)) if i % 2 else 0 for i in range(len(seqs))]
+    ext = [0 if i == 0 and len(seqs) > 1 else s for i, s in enumerate(seqs)]
+    total = [p + s for p, s in zip(pre, ext)]
+    last = [int(rng.integers(1, 100)) * ps + (p - 1) % ps if p else -1 for p in pre]
+    pages = sum(-(-t // ps) for t in total) + 5
+    free_pages = [int(x) for x in rng.permutation(np.arange(1, pages + 1))]
+    alloc = ref.PagedAllocator(num_pages=pages, page_size=ps)
+    alloc.free_pages = list(free_pages)
+    expect = alloc.alloc_extend(pre, total, last)
+    t = {k: torch.tensor(v, dtype=torch.int64, device=dev)
+         for k, v in dict(pre=pre, total=total, last=last, free=free_pages).items()}
+    out = torch.empty(sum(ext), dtype=torch.int64, device=dev)
+    rc = lib.load().atlas_alloc_extend_slots(lib.ptr(t["pre"]), lib.ptr(t["total"]), lib.ptr(t["last"]),
+                                             lib.ptr(t["free"]), ps, len(seqs), lib.ptr(out), lib.stream_of(dev))
+    lib.check(rc, "alloc_extend")
+    assert out.cpu().tolist() == expect
+
+
+@pytest.mark.parametrize("ps", [3, 64, 130])
+def test_paged_metadata_flags_any_bad_slot(dev, ps):
+    """One displaced slot anywhere in a page (each lane's first and later slots) clears the layout flag."""
+    pm = pkg("flashinfer_paged.paged_metadata")
+    good = _slot_path([5, 2, 9], 2 * ps + 1, ps)
+    for at in sorted({0, 1, ps - 1, ps, 2 * ps - 1, 2 * ps, min(64, ps), min(65, 2 * ps)}):
+        bad = list(good)
+        bad[at] += 1
+        md = pm.build_flashinfer_paged_kv_metadata([torch.tensor(p, device=dev) for p in (good, bad)], page_size=ps)
+        with pytest.raises(RuntimeError, match="page-aligned"):
+            md.assert_layout_valid()
+    pm.build_flashinfer_paged_kv_metadata([torch.tensor(good, device=dev)], page_size=ps, sync_check=True)
