@@ -11,7 +11,6 @@ namespace atlas {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kUnroll = 4;
 
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 
@@ -21,34 +20,22 @@ struct InlineItems {
   int32_t req[ATLAS_MAX_INLINE_ITEMS];
 };
 
-// K[dst] <- K[src], V[dst] <- V[src] for every layer of the table.
+// K[dst] <- K[src], V[dst] <- V[src] for every layer of the table, one vector
+// per thread.
 __global__ __launch_bounds__(kThreads) void kv_move_kernel(LayerTable lt, SlotGeom g,
                                                            const int64_t* __restrict__ dst,
                                                            const int64_t* __restrict__ src,
                                                            int64_t n) {
   const int layer = blockIdx.y >> 1;
   char* base = const_cast<char*>((blockIdx.y & 1) ? lt.v[layer] : lt.k[layer]);
-  const int64_t total = n * g.row_vecs;
-  const int64_t first = int64_t(blockIdx.x) * kThreads * kUnroll + threadIdx.x;
-  uint4 buf[kUnroll];
-  int64_t dofs[kUnroll];
-#pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int64_t idx = first + int64_t(u) * kThreads;
-    dofs[u] = -1;
-    if (idx < total) {
-      int64_t item;
-      int vec;
-      split_row(idx, g, item, vec);
-      const int64_t so = slot_offset(src[item], g) + vec_offset(vec, g);
-      dofs[u] = slot_offset(dst[item], g) + vec_offset(vec, g);
-      buf[u] = *reinterpret_cast<const uint4*>(base + so);
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    if (dofs[u] >= 0) *reinterpret_cast<uint4*>(base + dofs[u]) = buf[u];
-  }
+  const int64_t idx = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+  if (idx >= n * g.row_vecs) return;
+  int64_t item;
+  int vec;
+  split_row(idx, g, item, vec);
+  const int64_t so = slot_offset(src[item], g) + vec_offset(vec, g);
+  const int64_t dof = slot_offset(dst[item], g) + vec_offset(vec, g);
+  *reinterpret_cast<uint4*>(base + dof) = *reinterpret_cast<const uint4*>(base + so);
 }
 
 // One wave per moved slot, for rows of CPR 1 KiB chunks (1 KiB and 2 KiB
@@ -103,7 +90,15 @@ struct SrcTable {
   const char* v[ATLAS_MAX_LAYERS_PER_LAUNCH];
 };
 
-// Dense rows -> slots, every layer.
+// Dense rows -> slots, every layer.  UNROLL vectors per thread, branch-free:
+// vectors past the last one copy the last vector again (the same bytes to the
+// same place), so a thread's slot load and row loads are in flight together.
+// Small appends are bound by that chain of round trips, large ones by HBM.
+// (With a branch around each of four vectors the compiler waits for every
+// vector's loads before it issues the next one's: 200 rows of one layer took
+// 7.8 us and take 2.1, 72 rows of 16 layers 13.8 and 3.0.)  STREAM: loads and
+// stores carry the non-temporal hint, see kStreamBytes.
+template <int UNROLL, bool STREAM>
 __global__ __launch_bounds__(kThreads) void kv_append_kernel(LayerTable lt, SrcTable st, SlotGeom g,
                                                              int64_t src_token_stride,
                                                              const int64_t* __restrict__ dst,
@@ -113,25 +108,29 @@ __global__ __launch_bounds__(kThreads) void kv_append_kernel(LayerTable lt, SrcT
   char* base = const_cast<char*>(is_v ? lt.v[layer] : lt.k[layer]);
   const char* sbase = is_v ? st.v[layer] : st.k[layer];
   const int64_t total = n * g.row_vecs;
-  const int64_t first = int64_t(blockIdx.x) * kThreads * kUnroll + threadIdx.x;
-  uint4 buf[kUnroll];
-  int64_t dofs[kUnroll];
+  const int64_t first = int64_t(blockIdx.x) * kThreads * UNROLL + threadIdx.x;
+  int64_t item[UNROLL], slot[UNROLL];
+  int vec[UNROLL];
+  u32x4v buf[UNROLL];
 #pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    const int64_t idx = first + int64_t(u) * kThreads;
-    dofs[u] = -1;
-    if (idx < total) {
-      int64_t item;
-      int vec;
-      split_row(idx, g, item, vec);
-      const int64_t slot = dst ? dst[item] : dst_start + item;
-      dofs[u] = slot_offset(slot, g) + vec_offset(vec, g);
-      buf[u] = *reinterpret_cast<const uint4*>(sbase + item * src_token_stride + int64_t(vec) * 16);
-    }
+  for (int u = 0; u < UNROLL; ++u) {
+    split_row(min(first + int64_t(u) * kThreads, total - 1), g, item[u], vec[u]);
+    slot[u] = dst_start + item[u];
+  }
+  if (dst != nullptr) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) slot[u] = dst[item[u]];
   }
 #pragma unroll
-  for (int u = 0; u < kUnroll; ++u) {
-    if (dofs[u] >= 0) *reinterpret_cast<uint4*>(base + dofs[u]) = buf[u];
+  for (int u = 0; u < UNROLL; ++u) {
+    const u32x4v* p = reinterpret_cast<const u32x4v*>(sbase + item[u] * src_token_stride + int64_t(vec[u]) * 16);
+    buf[u] = STREAM ? __builtin_nontemporal_load(p) : *p;
+  }
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) {
+    u32x4v* p = reinterpret_cast<u32x4v*>(base + slot_offset(slot[u], g) + vec_offset(vec[u], g));
+    if (STREAM) __builtin_nontemporal_store(buf[u], p);
+    else *p = buf[u];
   }
 }
 
@@ -284,9 +283,9 @@ void fill_table(LayerTable& lt, const void* const* k_layers, const void* const* 
   }
 }
 
-dim3 copy_grid(int64_t n, const SlotGeom& g, int nl) {
+dim3 copy_grid(int64_t n, const SlotGeom& g, int nl, int unroll) {
   const int64_t total = n * g.row_vecs;
-  const int64_t per_block = int64_t(kThreads) * kUnroll;
+  const int64_t per_block = int64_t(kThreads) * unroll;
   return dim3(static_cast<unsigned>((total + per_block - 1) / per_block), static_cast<unsigned>(2 * nl));
 }
 
@@ -323,12 +322,19 @@ extern "C" int atlas_kv_move_slots(const void* const* k_layers, const void* cons
       if ((rc = launch_status("kv_move_rows_kernel"))) return rc;
       continue;
     }
-    hipLaunchKernelGGL(kv_move_kernel, copy_grid(n, g, nl), dim3(kThreads), 0,
+    hipLaunchKernelGGL(kv_move_kernel, copy_grid(n, g, nl, 1), dim3(kThreads), 0,
                        static_cast<hipStream_t>(stream), lt, g, dst_slots_dev, src_slots_dev, n);
     if ((rc = launch_status("kv_move_kernel"))) return rc;
   }
   return ATLAS_OK;
 }
+
+// From this many bytes of one launch's rows on, an append streams: they are
+// more than the L2s hold (32 MB).  16 layers of 1 KiB rows: 1000 rows (33 MB)
+// 13.5 us streamed against 15.4, 4848 rows 52.9 (6.0 TB/s) against 58.4, but 500
+// rows 8.0 against 7.7; before, four branched vectors per thread, 27.8, 73.1
+// and 21.8.
+constexpr int64_t kStreamBytes = int64_t(32) << 20;
 
 extern "C" int atlas_kv_append(const void* const* k_layers, const void* const* v_layers,
                                int num_layers, int64_t page_size, int64_t page_stride,
@@ -356,9 +362,12 @@ extern "C" int atlas_kv_append(const void* const* k_layers, const void* const* v
       st.k[i] = i < nl ? static_cast<const char*>(k_src[l0 + i]) : nullptr;
       st.v[i] = i < nl ? static_cast<const char*>(v_src[l0 + i]) : nullptr;
     }
-    hipLaunchKernelGGL(kv_append_kernel, copy_grid(n, g, nl), dim3(kThreads), 0,
-                       static_cast<hipStream_t>(stream), lt, st, g, src_token_stride, dst_slots_dev,
-                       dst_start, n);
+    if (n * row_bytes * 2 * nl >= kStreamBytes)
+      hipLaunchKernelGGL((kv_append_kernel<2, true>), copy_grid(n, g, nl, 2), dim3(kThreads), 0,
+                         static_cast<hipStream_t>(stream), lt, st, g, src_token_stride, dst_slots_dev, dst_start, n);
+    else
+      hipLaunchKernelGGL((kv_append_kernel<1, false>), copy_grid(n, g, nl, 1), dim3(kThreads), 0,
+                         static_cast<hipStream_t>(stream), lt, st, g, src_token_stride, dst_slots_dev, dst_start, n);
     if ((rc = launch_status("kv_append_kernel"))) return rc;
   }
   return ATLAS_OK;

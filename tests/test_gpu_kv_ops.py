@@ -444,3 +444,40 @@ def test_hnd_layout_geometry_and_refusals(dev):
     assert nhd_geom.token_stride == 8 * 256 and nhd_geom.head_stride == 256
     with pytest.raises(ValueError, match="kv_layout"):
         kv.paged_layer_geometry(hnd, "NDH")
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025])
+def test_append_token_pool_streamed_and_cached(dev, n):
+    """Appends on both sides of the byte limit from which the rows are streamed (32 MiB: 1024 rows of 1 KiB, K and
+    V of 16 layers), bit for bit; slots outside the list keep their rows."""
+    kv = pkg("kv_ops")
+    gen = torch.Generator(device=dev).manual_seed(n)
+    layers, h, d, slots = 16, 8, 64, 1100
+
+    def rows(count):
+        return torch.randint(-2 ** 15, 2 ** 15, (2, layers, count, h, d), generator=gen, device=dev,
+                             dtype=torch.int16).view(torch.float16)
+
+    pool, src = rows(slots), rows(n)
+    dst = torch.randperm(slots, generator=gen, device=dev)[:n]
+    expect = pool.clone().view(torch.int16)
+    expect[:, :, dst] = src.view(torch.int16)
+    kv.append_token_pool(list(pool[0]), list(pool[1]), list(src[0]), list(src[1]), dst)
+    assert torch.equal(pool.view(torch.int16), expect)
+
+
+@pytest.mark.parametrize("n,dim", [(1, 8), (33, 24), (40, 40)])
+def test_move_slots_general_rows(dev, n, dim):
+    """Rows that are not 1 or 2 KiB move one vector per thread."""
+    kv = pkg("kv_ops")
+    gen = torch.Generator().manual_seed(dim)
+    k, v = ([_rand(gen, (128, 4, dim), torch.float16).to(dev) for _ in range(3)] for _ in range(2))
+    perm = torch.randperm(128, generator=gen)
+    src, dst = perm[:n], perm[64:64 + n]
+    expect = []
+    for t in k + v:
+        e = t.cpu().clone()
+        e[dst] = e[src]
+        expect.append(e)
+    kv.move_slots(k, v, dst.to(dev), src.to(dev))
+    assert all(torch.equal(t.cpu(), e) for t, e in zip(k + v, expect))
