@@ -50,15 +50,16 @@ struct Vec {
 };
 
 // Workgroup (c, r) reads chunk c of logits row r once: the chunk's maximum m
-// and the sum of exp(x - m), kept online per thread (16-byte loads when the
-// rows are 16-byte aligned), then reduced over the workgroup.  It stores the
-// pair into its slot of the row and counts itself in on the row's arrival
-// counter with one agent-scope read-modify-write that releases the slot; the
-// workgroup that arrives last (the counter held num_chunks - 1) acquires
-// every slot, combines the pairs in chunk order (a fixed order, so the LSE is
-// the same on every run), writes the row LSE and every gather of row r, and
-// empties the slots and the counter for the next call.  A slot is
-// (max bits, ~sum bits); every slot is written before its workgroup arrives.
+// and the sum of exp(x - m), kept online per thread over batches of kBatch
+// 16-byte loads, then reduced over the
+// workgroup.  It stores the pair into its slot of the row, waits until the
+// store is acknowledged and counts itself in on the row's arrival counter; the
+// workgroup that arrives last (the counter held num_chunks - 1) reads every
+// slot, combines the pairs in chunk order (a fixed order, so the LSE is the same
+// on every run), writes the row LSE and every gather of row r, and empties the
+// slots and the counter for the next call.  A slot is (max bits, ~sum bits).
+// Slots and counters are agent-scope atomics, which every XCD sees, so no
+// workgroup needs a release (a write-back of its XCD's whole L2).
 struct GatherArgs {
   const char* logits;
   int64_t row_stride_bytes;
@@ -79,7 +80,8 @@ struct GatherArgs {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-constexpr int kPre = 2;  // gathers per thread whose logits are loaded ahead of the combine
+constexpr int kPre = 2;    // gathers per thread whose logits are loaded ahead of the combine
+constexpr int kBatch = 4;  // 16-byte loads a thread has in flight (8 measured slower: 26.9 us against 24.1)
 
 // (m, s) pairs: s is a sum of exp(x - m).
 __device__ __forceinline__ void pair_merge(float& m, float& s, float m2, float s2) {
@@ -89,7 +91,30 @@ __device__ __forceinline__ void pair_merge(float& m, float& s, float m2, float s
   m = mn;
 }
 
-template <int DT, bool VEC>
+// Adds N vectors to a thread's (m, s).
+template <int DT, int N>
+__device__ __forceinline__ void batch_add(const Vec<DT> (&x)[N], float& m, float& s) {
+  constexpr int EPV = Vec<DT>::kElems;
+  float mn = m;
+#pragma unroll
+  for (int b = 0; b < N; ++b)
+#pragma unroll
+    for (int k = 0; k < EPV; k += 2)  // one three-input maximum per two logits (a NaN stays and ends in the sum)
+      mn = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mn, x[b].x[k]), x[b].x[k + 1]);
+  const float mb = mn == -INFINITY ? 0.f : mn * kLog2e;  // (all -inf so far: adds zeros)
+  float acc = m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - mn) * kLog2e);
+#pragma unroll
+  for (int b = 0; b < N; ++b) {
+    float part = 0.f;
+#pragma unroll
+    for (int k = 0; k < EPV; ++k) part += __builtin_amdgcn_exp2f(__builtin_fmaf(x[b].x[k], kLog2e, -mb));
+    acc += part;
+  }
+  m = mn;
+  s = acc;
+}
+
+template <int DT>
 __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a) {
   __shared__ float red_m[kThreads / 64];
   __shared__ float red_s[kThreads / 64];
@@ -115,41 +140,43 @@ __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a)
     gtok[k] = a.n > 0 ? a.tokens[i] : 0;
   }
 
+  // 16-byte loads over the chunk's aligned part [a0, a1); at most EPV - 1 single
+  // elements before it and after it (rows of an odd vocabulary start anywhere).
+  constexpr int ES = DT == ATLAS_DTYPE_F32 ? 4 : 2;
+  const int lead = static_cast<int>((-reinterpret_cast<uintptr_t>(row + c0 * ES) & 15) / ES);
+  const int64_t a0 = min(c1, c0 + lead);
+  const int64_t nv = (c1 - a0) / EPV;
+  const int64_t a1 = a0 + nv * EPV;
+  const char* vrow = row + a0 * ES;
   float m = -INFINITY, s = 0.f;
-  int64_t scalar0 = c0;
-  if constexpr (VEC) {
-    // whole vectors of the chunk (chunk starts are multiples of 8 elements)
-    const int64_t v0 = c0 / EPV;
-    const int64_t v1 = c1 / EPV;
-    scalar0 = v1 * EPV;
-#pragma unroll 4
-    for (int64_t v = v0 + t; v < v1; v += kThreads) {
-      Vec<DT> x;
-      x.load(row + v * 16);
-      float vm = x.x[0];
+  int64_t v = t;
+  // full batches: one running maximum and one rescale per kBatch vectors
+  for (; v + int64_t(kBatch - 1) * kThreads < nv; v += int64_t(kBatch) * kThreads) {
+    Vec<DT> x[kBatch];
 #pragma unroll
-      for (int k = 1; k < EPV; ++k) vm = fmaxf(vm, x.x[k]);
-      const float mn = fmaxf(m, vm);
-      float acc = m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - mn) * kLog2e);
-      const float mb = mn == -INFINITY ? 0.f : mn * kLog2e;  // (an all -inf vector adds zeros)
-#pragma unroll
-      for (int k = 0; k < EPV; ++k) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(x.x[k], kLog2e, -mb));
-      m = mn;
-      s = acc;
-    }
+    for (int b = 0; b < kBatch; ++b) x[b].load(vrow + (v + int64_t(b) * kThreads) * 16);
+    batch_add<DT, kBatch>(x, m, s);
   }
-  for (int64_t i = scalar0 + t; i < c1; i += kThreads) {
-    const float x = load_logit<DT>(row, i);
-    pair_merge(m, s, x, 1.f);
+  for (; v < nv; v += kThreads) {
+    Vec<DT> x[1];
+    x[0].load(vrow + v * 16);
+    batch_add<DT, 1>(x, m, s);
   }
-  // The gathered logits go out now and land while the pair is published.
+  const int singles = static_cast<int>((a0 - c0) + (c1 - a1));
+  if (t < singles) {
+    const int64_t i = t < a0 - c0 ? c0 + t : a1 + (t - (a0 - c0));
+    pair_merge(m, s, load_logit<DT>(row, i), 1.f);
+  }
+  // The gathered logits go out now and land while the pair is published.  Lanes
+  // whose gather belongs to another row read the chunk's first logit instead: a
+  // read at their own token would fetch a line of this row that nobody needs.
   float gx[kPre];
   bool gmine[kPre];
 #pragma unroll
   for (int k = 0; k < kPre; ++k) {
     gmine[k] = t + int64_t(k) * kThreads < a.n && grow[k] == r;
     const bool ok = gtok[k] >= 0 && gtok[k] < a.vocab;
-    gx[k] = load_logit<DT>(row, ok ? gtok[k] : 0);
+    gx[k] = load_logit<DT>(row, gmine[k] && ok ? gtok[k] : c0);
     if (!ok) gx[k] = NAN;
   }
   // workgroup reduction of (m, s)
@@ -166,12 +193,17 @@ __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a)
 #pragma unroll
     for (int w = 1; w < kThreads / 64; ++w) pair_merge(bm, bs, red_m[w], red_s[w]);
     const uint64_t slot = uint64_t(__float_as_uint(bm)) | (uint64_t(~__float_as_uint(bs)) << 32);
-    __hip_atomic_store(rs + c, slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // The release orders the slot before the arrival; the last arriver's
-    // acquire then sees every slot (all earlier arrivals released theirs).
-    const uint32_t prev = __hip_atomic_fetch_add(a.arrivals + r, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    const bool last = prev == uint32_t(a.num_chunks - 1);
-    if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    bool last = true;
+    if (a.num_chunks > 1) {
+      __hip_atomic_store(rs + c, slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // The slot's store is acknowledged before the arrival goes out, so the
+      // last arriver's loads, issued behind its own arrival, find every slot.
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const uint32_t prev = __hip_atomic_fetch_add(a.arrivals + r, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = prev == uint32_t(a.num_chunks - 1);
+    } else {
+      lse_sh = bm + __builtin_log2f(bs) * kLn2;
+    }
     last_sh = last;
   }
   __syncthreads();
@@ -179,7 +211,7 @@ __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a)
 
   // The last arriver: combine the row's slots in chunk order (one per lane of
   // wave 0, then a fixed pairwise tree).
-  if (t < 64) {
+  if (t < 64 && a.num_chunks > 1) {
     float cm = -INFINITY, cs = 0.f;
     for (int k = t; k < a.num_chunks; k += 64) {
       const uint64_t v = __hip_atomic_load(rs + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -191,12 +223,12 @@ __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a)
   }
   __syncthreads();
   const float lse = lse_sh;
-  if (t == 0) {
-    if (a.row_lse) a.row_lse[r] = lse;
-    __hip_atomic_store(a.arrivals + r, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (t == 0 && a.row_lse) a.row_lse[r] = lse;
+  if (a.num_chunks > 1) {
+    if (t == 0) __hip_atomic_store(a.arrivals + r, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = t; k < a.num_chunks; k += kThreads)
+      __hip_atomic_store(rs + k, uint64_t(0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  for (int k = t; k < a.num_chunks; k += kThreads)
-    __hip_atomic_store(rs + k, uint64_t(0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
   for (int k = 0; k < kPre; ++k)
     if (gmine[k]) a.out[t + int64_t(k) * kThreads] = gx[k] - lse;
@@ -215,21 +247,23 @@ using namespace atlas;
 namespace atlas {
 namespace {
 // Chunks per row: about ATLAS_GATHER_TARGET_WGS (row, chunk) workgroups in
-// all, chunks of at least 1024 logits, at most 256 chunks per row.  Every
-// workgroup ends with an agent-scope release (the L2 write-back that orders
-// its slot before its arrival), so fewer, longer chunks win: 35 rows x 128256
-// fp16 logits take 8.4 us with 128 workgroups, 9.0 with 256 and 10.4 with 512
-// (9.3 with 64 and 12.4 with one workgroup per row).
+// all, chunks of at least kMinChunk logits (two full batches), at most 256
+// chunks per row.  A workgroup costs its reduction and its arrival, so one per
+// CU is enough: 416 rows x 128256 bf16 logits in one chunk each take 23.8 us
+// (4.5 TB/s), in two 27.5 and in five 25.8; 35 rows in eight chunks 8.3 us, in
+// sixteen 10.1.  (Each workgroup with an L2 write-back at its end, and every
+// lane reading its gather's token in every row: 42.4 and 9.5 us.)
+constexpr int64_t kMinChunk = 16384;
 struct GatherGeom {
   int num_chunks;
   int64_t chunk_len;
 };
 #ifndef ATLAS_GATHER_TARGET_WGS
-#define ATLAS_GATHER_TARGET_WGS 128
+#define ATLAS_GATHER_TARGET_WGS 256
 #endif
 GatherGeom gather_geom(int64_t num_rows, int64_t vocab) {
   const int64_t want = (ATLAS_GATHER_TARGET_WGS + num_rows - 1) / num_rows;
-  const int64_t by_len = (vocab + 1023) / 1024;
+  const int64_t by_len = (vocab + kMinChunk - 1) / kMinChunk;
   int64_t chunks = std::max<int64_t>(1, std::min<int64_t>({want, by_len, 256}));
   int64_t len = (vocab + chunks - 1) / chunks;
   len = (len + 7) / 8 * 8;
@@ -284,22 +318,11 @@ extern "C" int atlas_gather_logprobs(const void* logits_dev, int64_t row_stride,
   a.chunk_len = g.chunk_len;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(g.num_chunks), static_cast<unsigned>(total_rows));
-  const bool vec = (reinterpret_cast<uintptr_t>(logits_dev) % 16) == 0 && a.row_stride_bytes % 16 == 0 &&
-                   (num_rows2 == 0 ||
-                    ((reinterpret_cast<uintptr_t>(logits2_dev) % 16) == 0 && a.row_stride2_bytes % 16 == 0));
-#define ATLAS_GATHER_LAUNCH(DT)                                                                          \
-  do {                                                                                                   \
-    if (vec)                                                                                             \
-      hipLaunchKernelGGL((gather_logprobs_kernel<DT, true>), grid, dim3(kThreads), 0, s, a);             \
-    else                                                                                                 \
-      hipLaunchKernelGGL((gather_logprobs_kernel<DT, false>), grid, dim3(kThreads), 0, s, a);            \
-  } while (0)
   if (dtype == ATLAS_DTYPE_F32)
-    ATLAS_GATHER_LAUNCH(ATLAS_DTYPE_F32);
+    hipLaunchKernelGGL((gather_logprobs_kernel<ATLAS_DTYPE_F32>), grid, dim3(kThreads), 0, s, a);
   else if (dtype == ATLAS_DTYPE_F16)
-    ATLAS_GATHER_LAUNCH(ATLAS_DTYPE_F16);
+    hipLaunchKernelGGL((gather_logprobs_kernel<ATLAS_DTYPE_F16>), grid, dim3(kThreads), 0, s, a);
   else
-    ATLAS_GATHER_LAUNCH(ATLAS_DTYPE_BF16);
-#undef ATLAS_GATHER_LAUNCH
+    hipLaunchKernelGGL((gather_logprobs_kernel<ATLAS_DTYPE_BF16>), grid, dim3(kThreads), 0, s, a);
   return launch_status("gather_logprobs_kernel");
 }

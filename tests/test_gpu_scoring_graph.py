@@ -273,3 +273,25 @@ def test_gather_logprobs_graph_replays(dev):
             lp_p = osc.log_softmax(prefix.float().cpu().double().numpy())
             exp = np.array([lp_p[0, t] if r == rows1 else lp_v[r, t] for r, t in zip(row_list, tok_list)])
             assert np.abs(eager.cpu().numpy() - exp).max() <= 2e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,vocab,offset", [(1, 16384, 0), (1, 16385, 1), (3, 32001, 3), (300, 4099, 1),
+                                               (2, 128256, 0)])
+def test_gather_logprobs_chunk_edges(dev, dtype, rows, vocab, offset):
+    """One chunk and several, chunks that end inside a 16-byte load, rows that start at every alignment, and rows
+    with -inf runs longer than a thread's batch, against float64 (fp32 sums of at most 2^17 exponentials in a
+    tree of batches: far below the 1e-5 allowed)."""
+    tr = pkg("target_runtime")
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    flat = torch.randn(rows * vocab + offset, generator=gen, device=dev, dtype=torch.float32).mul_(3).to(dtype)
+    logits = flat[offset:].view(rows, vocab)
+    logits[0, : vocab // 2] = float("-inf")
+    at = [r for r in range(rows) for _ in range(3)]
+    toks = [t for r in range(rows) for t in (vocab - 1, vocab // 2, (r * 7919) % vocab)]
+    got = tr.gather_token_logprobs(logits, at, toks)
+    x = logits.double()
+    expect = x[at, toks] - torch.logsumexp(x, dim=-1)[at]
+    finite = torch.isfinite(expect)
+    assert torch.equal(torch.isfinite(got), finite)
+    assert (got.double() - expect)[finite].abs().max().item() <= 1e-5 * expect[finite].abs().max().item()
