@@ -640,13 +640,15 @@ struct MergeArgs {
 
 // One wave per packed row, four rows per workgroup.  Lane (g, c) folds the
 // 16-byte chunk c of splits g, g + G, g + 2G, ... (G = 64 / (D / 8) split
-// groups) online, kMergeUnroll splits per round of independent loads (one
-// round covers 32 splits at head_dim 128); the groups then combine through
-// cross-lane reductions.  No LDS and no workgroup barriers, so a row costs
-// the merge item load and one round of partial-state loads.
+// groups) online, U splits per round of independent loads; the groups then
+// combine through cross-lane reductions.  No LDS and no workgroup barriers, so
+// a row costs the merge item load and one round of partial-state loads.  U is 8
+// (32 splits at head_dim 128 in one round), or 2 or 4 where that covers every
+// split: rounds of 8 issue loads that few splits have no use for (6 splits of
+// 200 nodes: 6.8 us with rounds of 8, 4.9 with 2; a decode step's cascade merge
+// 0.9 us less per layer).
 constexpr int kMergeThreads = 256;
 constexpr int kMergeRowsPerBlock = kMergeThreads / 64;
-constexpr int kMergeUnroll = 8;
 
 // Eight 16-bit values (fp16 or bf16) to floats.
 template <bool BF16>
@@ -678,7 +680,7 @@ __device__ __forceinline__ float group_sum(float v) {
 
 // Merges the split states of packed row `row` of merge item `mi` and writes
 // the final output row (and LSE), one wave per row.
-template <int D, bool BF16>
+template <int D, bool BF16, int U>
 __device__ __forceinline__ void merge_row(const MergeArgs& a, const atlas_attn_merge_t& mi, int row, int lane) {
   typedef Mfma<BF16> M;
   constexpr int CH = D / 8;   // 16-byte chunks per row
@@ -688,14 +690,18 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, const atlas_attn_m
   const int c = lane % CH;
   const int ns = mi.num_splits;
   const int64_t base = int64_t(mi.partial_row) + row;
+  const int qo_start = a.qo_indptr[mi.req];  // requested ahead of the partial rows
+  const int prow_q = mi.row_start + row;
+  const int node = prow_q / a.group;
+  const int head = mi.kv_head * a.group + (prow_q - node * a.group);
 
   float m_t = -INFINITY, wsum = 0.f;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int s0 = g; s0 < ns; s0 += kMergeUnroll * G) {
-    float l[kMergeUnroll];
-    uint4 raw[kMergeUnroll];
+  for (int s0 = g; s0 < ns; s0 += U * G) {
+    float l[U];
+    uint4 raw[U];
 #pragma unroll
-    for (int k = 0; k < kMergeUnroll; ++k) {
+    for (int k = 0; k < U; ++k) {
       // Splits past the last re-read split s0 (always present) and are
       // given weight zero: unconditional loads stay in one batch, where a
       // guarded load would be followed by a wait of its own.
@@ -707,7 +713,7 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, const atlas_attn_m
     }
     float m_new = m_t;
 #pragma unroll
-    for (int k = 0; k < kMergeUnroll; ++k) m_new = max2f(m_new, l[k]);
+    for (int k = 0; k < U; ++k) m_new = max2f(m_new, l[k]);
     // No early exit on an all-masked round: a branch here would hold the O
     // loads back behind the LSE loads.  With m_new = -inf every weight is 0.
     const float sc = m_t == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_t - m_new);
@@ -715,7 +721,7 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, const atlas_attn_m
     for (int i = 0; i < 8; ++i) acc[i] *= sc;
     wsum *= sc;
 #pragma unroll
-    for (int k = 0; k < kMergeUnroll; ++k) {
+    for (int k = 0; k < U; ++k) {
       const float wk = l[k] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(l[k] - m_new);
       float v[8];
       unpack8<BF16>(raw[k], v);
@@ -732,10 +738,6 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, const atlas_attn_m
   for (int i = 0; i < 8; ++i) acc[i] = group_sum<CH>(acc[i] * f);
   if (g != 0) return;
   const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-  const int prow_q = mi.row_start + row;
-  const int node = prow_q / a.group;
-  const int head = mi.kv_head * a.group + (prow_q - node * a.group);
-  const int qo_start = a.qo_indptr[mi.req];
   char* orow = a.out + ((int64_t(qo_start + node) * a.out_stride_token + int64_t(head) * a.out_stride_head) * 2);
   uint32_t pk[4];
 #pragma unroll
@@ -754,7 +756,11 @@ __global__ __launch_bounds__(kMergeThreads) void tree_attn_merge_kernel(MergeArg
   const int row = blockIdx.y * kMergeRowsPerBlock + (threadIdx.x >> 6);
   if (row >= mi.num_rows) return;
   if (mi.partial_row < 0 || int64_t(mi.partial_row) + int64_t(mi.num_splits) * mi.num_rows > a.part_rows) return;
-  merge_row<D, BF16>(a, mi, row, threadIdx.x & 63);
+  constexpr int G = 64 / (D / 8);
+  const int lane = threadIdx.x & 63;
+  if (mi.num_splits <= 2 * G) merge_row<D, BF16, 2>(a, mi, row, lane);
+  else if (mi.num_splits <= 4 * G) merge_row<D, BF16, 4>(a, mi, row, lane);
+  else merge_row<D, BF16, 8>(a, mi, row, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -798,22 +804,23 @@ __device__ __forceinline__ void wait_vmcnt() {
 // Issued as inline assembly so the compiler's wait-count pass, which would
 // wait for every outstanding load before each LDS read, leaves the ring's
 // in-flight tiles alone; the kernel waits for them explicitly (wait_vmcnt).
+// A load to LDS needs one wait state after the write of m0.
 __device__ __forceinline__ void dma16(const char* gaddr, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gaddr), "s"(lds_base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gaddr), "s"(lds_base) : "memory", "m0");
 }
 
 // KV rows are read once per launch, so their loads carry the non-temporal
 // hint: they do not displace the queries, page ids and partial rows from the
 // caches (1.2 us per layer less on the 16k forest).
 __device__ __forceinline__ void dma16_kv(const char* gaddr, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(gaddr), "s"(lds_base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(gaddr), "s"(lds_base) : "memory", "m0");
 }
 
 // The KV load with a wave-uniform 64-bit base in SGPRs and a 32-bit per-lane
 // offset: the base's arithmetic runs on the scalar unit, the offsets stay in
 // registers for the whole loop.
 __device__ __forceinline__ void dma16_s(const char* sbase, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase), "s"(lds_base)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase), "s"(lds_base)
                : "memory", "m0");
 }
 
