@@ -122,6 +122,10 @@ struct Mfma<false> {
   static __device__ __forceinline__ uint32_t pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
   }
+  // Two values rounded to nearest.
+  static __device__ __forceinline__ uint32_t round2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, half2v{static_cast<_Float16>(a), static_cast<_Float16>(b)});
+  }
   static __device__ __forceinline__ float sum2(uint32_t packed, float acc) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, packed), half2v{(_Float16)1.0f, (_Float16)1.0f}, acc,
                                   false);
@@ -148,6 +152,7 @@ struct Mfma<true> {
   static __device__ __forceinline__ uint32_t pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, bf16x2v{static_cast<__bf16>(a), static_cast<__bf16>(b)});
   }
+  static __device__ __forceinline__ uint32_t round2(float a, float b) { return pack2(a, b); }
   static __device__ __forceinline__ float sum2(uint32_t packed, float acc) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2v, packed),
                                            bf16x2v{(__bf16)1.0f, (__bf16)1.0f}, acc, false);
@@ -1398,6 +1403,14 @@ __device__ __forceinline__ void d128_loop(RowState<BF16, RT>& st, Ring<NL>& r, c
   }
 }
 
+// 16 bytes stored with agent scope (the store instruction of a relaxed
+// agent-scope atomic, at twice its width).  A store of more than 8 bytes still
+// reads its data one wait state later, which the compiler cannot see here.
+__device__ __forceinline__ void store16_agent(char* dst, u32x4v v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(dst), "v"(v) : "memory");
+}
+typedef uint32_t u32x4a8 __attribute__((ext_vector_type(4), aligned(8)));  // output rows are only 8-byte aligned
+
 // Writes one finished row (the final output, or the split's partial state,
 // both in the output dtype) for the lanes' D columns 16*dt + 4*grp .. +3, dt
 // in [dt0, dt0 + NDT).
@@ -1407,29 +1420,40 @@ __device__ __forceinline__ void d128_store(const AttnArgs& a, const atlas_attn_w
                                            float inv, float lse2, bool write_lse, int grp) {
   typedef Mfma<BF16> M;
   constexpr int D = 128;
-  if (!row_ok) return;
   const bool final_row = w.partial_row < 0;
   const int64_t prow = int64_t(w.partial_row) + lrow;
-  if (!final_row && prow >= a.part_rows) return;
+  // (a row's four lanes agree, but every lane takes part in the swaps below)
+  const bool store = row_ok && (final_row || prow < a.part_rows);
   char* orow = final_row ? a.out + ((int64_t(c.qo_start + node) * a.out_stride_token +
                                      int64_t(head) * a.out_stride_head) * 2)
                          : reinterpret_cast<char*>(a.part_o + prow * D);
+  // Two 16-dim blocks at a time: the lanes of an even and an odd group swap
+  // halves, so a lane holds eight consecutive dims (even groups of the first
+  // block, odd groups of the second) and a row's 64 bytes go out as four
+  // 16-byte stores (the end of a wave with one row tile of the 16k forest:
+  // 0.96 us, with 8-byte stores 1.56).
   // Split partial rows are written through to memory (agent-scope stores):
   // the merge launch reads them from other XCDs, and nothing of them is left
   // dirty in this XCD's L2 at the end of the launch (0.3 us per layer less
   // on the 16k forest).
 #pragma unroll
-  for (int i = 0; i < NDT; ++i) {
-    const int dt = dt0 + i;
-    const uint32_t lo = uint32_t(M::from_float(o[i][0] * inv)) | (uint32_t(M::from_float(o[i][1] * inv)) << 16);
-    const uint32_t hi = uint32_t(M::from_float(o[i][2] * inv)) | (uint32_t(M::from_float(o[i][3] * inv)) << 16);
-    char* dst = orow + (dt * 16 + grp * 4) * 2;
-    if (final_row)
-      *reinterpret_cast<uint2*>(dst) = uint2{lo, hi};
-    else
-      __hip_atomic_store(reinterpret_cast<uint64_t*>(dst), uint64_t(lo) | (uint64_t(hi) << 32), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+  for (int i = 0; i < NDT; i += 2) {
+    uint32_t p[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      p[h][0] = M::round2(o[i + h][0] * inv, o[i + h][1] * inv);
+      p[h][1] = M::round2(o[i + h][2] * inv, o[i + h][3] * inv);
+    }
+    const auto lo = __builtin_amdgcn_permlane16_swap(p[0][0], p[1][0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(p[0][1], p[1][1], false, false);
+    const u32x4v v = {lo[0], hi[0], lo[1], hi[1]};
+    char* dst = orow + ((dt0 + i + (grp & 1)) * 16 + (grp >> 1) * 8) * 2;
+    if (store) {
+      if (final_row) *reinterpret_cast<u32x4a8*>(dst) = v;
+      else store16_agent(dst, v);
+    }
   }
+  if (!store) return;
   if (write_lse && grp == 0) {
     if (!final_row) __hip_atomic_store(a.part_lse + prow, lse2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else if (a.lse != nullptr) a.lse[int64_t(c.qo_start + node) * a.num_qo_heads + head] = lse2 * kLn2;
