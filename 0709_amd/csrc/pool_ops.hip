@@ -241,7 +241,7 @@ __global__ __launch_bounds__(kSweepThreads) void prune_paths_gather_kernel(
 // and every later slot of the page (within the path length) to follow it
 // contiguously, each lane checking every lanes-th slot of its page.
 // Bound by latency: a page's slots are one round of coalesced loads (8 prompts
-// of 4.8k tokens, pages of 64: 3.0 us; with one thread walking a page's slots,
+// of 4.8k tokens in all, pages of 64: 4.3 us; with one thread walking a page's slots,
 // each load behind the last one's compare, 12.3 us).
 __global__ __launch_bounds__(256) void paged_metadata_kernel(const int64_t* slots, const int64_t* path_offsets,
                                                              const int64_t* page_offsets, int num_paths,
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(1024) void alloc_decode_kernel(const int64_t* seq_l
 // thread; a request's token and page offsets are the sums over the requests
 // before it, which the workgroup reads for itself, so the host uploads nothing.
 // Bound by latency: two rounds of dependent loads (8 prompts of 4.8k tokens:
-// 4.4 us; one thread per request walking its tokens took 141 us, a store and a
+// 4.3 us; one thread per request walking its tokens took 141 us, a store and a
 // possible load per token in series).
 constexpr int kExtendThreads = 256;
 

@@ -979,9 +979,10 @@ def test_tree_spec_upload_copies_and_fills(dev, source):
 @pytest.mark.parametrize("splits", [2, 8, 9, 16, 17, 32, 33])
 def test_merge_rounds_cover_every_split(dev, d, dtype, splits):
     """The merge folds 2, 4 or 8 splits per lane and round (4 split groups at head_dim 128, 8 at 64): split counts
-    at and past the edge of each, all of equal weight, so that a split left out or folded twice shows.  (bf16: P and
-    O carry 8 bits, 2^-8 of outputs of at most 0.1 x 4 deviations, and the same once more for the partial rows.)"""
-    c = _build(dev, seed=splits, prefix_len=64 * 33 - 5, routes=[(1, 2), (3, 4)], d=d, dtype=dtype)
+    at and past the edge of each, one tile per split, all of about equal weight, so that a split left out or folded
+    twice shows.  (bf16: P and O carry 8 bits, 2^-8 of outputs of at most 0.1 x 4 deviations, and the same once more
+    for the partial rows.)"""
+    c = _build(dev, seed=splits, prefix_len=64 * splits - 10, routes=[(1, 2), (3, 4)], d=d, dtype=dtype)
     w, _, _ = _run_and_check(dev, c, split_target=8 * splits, atol=ATOL if dtype == torch.float16 else 4e-3)
     plan = w.current_plan
     assert plan.num_merge == 8 and plan.num_work == 8 * splits
