@@ -1479,7 +1479,8 @@ __device__ __forceinline__ void d128_store_rows(RowState<BF16, RT>& st, const At
 // the tile's first part): each part's unnormalised O, running max and row sum
 // go to LDS; after a workgroup barrier, part p combines the S states for D
 // columns [128 p / S, 128 (p + 1) / S) and stores them.  The caller's barriers
-// bracket the LDS exchange (every wave of the workgroup takes part in them).
+// bracket the LDS exchange (every wave of the workgroup takes part in them); the
+// one after the parts are written waits for those writes, as a bare one does not.
 constexpr int kPartBytes = 8 * 64 * 16 + 2 * 64 * 4;  // O^T accumulators, then m and l per lane
 
 template <bool BF16>
@@ -1558,7 +1559,7 @@ __device__ __forceinline__ void d128_item_split(const AttnArgs& a, const atlas_a
       ring_only<NL>(r, a, w, c, T);
     }
     bare_barrier();
-    bare_barrier();
+    __syncthreads();
     return;
   }
   const int j = wave - 4;
@@ -1570,7 +1571,7 @@ __device__ __forceinline__ void d128_item_split(const AttnArgs& a, const atlas_a
     d128_loop<BF16, NL, 1, 1, false>(st, r, a, c, lds, j, lane);
     bare_barrier();
     d128_part_put<BF16>(st, lds, j, lane);
-    bare_barrier();
+    __syncthreads();
     d128_part_merge<BF16, 4>(st, lds, 0, j, a, w, c, lane);
   } else {
     d128_load_rows<BF16, 1>(st, a, w, c, 4 * k + (j >> 1), 0, lane);
@@ -1579,7 +1580,7 @@ __device__ __forceinline__ void d128_item_split(const AttnArgs& a, const atlas_a
     d128_loop<BF16, NL, 1, 2, false>(st, r, a, c, lds, 2 * (j & 1), lane);
     bare_barrier();
     d128_part_put<BF16>(st, lds, j, lane);
-    bare_barrier();
+    __syncthreads();
     d128_part_merge<BF16, 2>(st, lds, j & ~1, j & 1, a, w, c, lane);
   }
 }
