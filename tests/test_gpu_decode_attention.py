@@ -330,3 +330,12 @@ def test_hnd_pages_equal_nhd_pages(dev, d, ps, cascade, as_tuple):
                                    last)
     assert float(np.abs(on.float().numpy() - ro).max()) <= ATOL
     assert float(np.abs(ln.numpy() - rl).max()) <= ATOL
+
+
+@pytest.mark.parametrize("ps", [1, 2, 3, 4, 8, 64, 128])
+@pytest.mark.parametrize("extra", [(1, 3), (60, 68)])
+def test_page_sizes_on_both_sides_of_the_branch_free_staging(dev, ps, extra):
+    """head_dim 64 stages pages of a power of two >= 2 without branches and other page sizes with them: odd and even
+    lengths around one and two 64-key tiles, whose last thread's second key lies past the end."""
+    _check(dev, seed=ps, requests=3, routes=3, prefix_range=(2 * ps, 4 * ps + 70), extra_range=extra, hq=8, hkv=2,
+           d=64, ps=ps, dtype=torch.float16)
