@@ -141,12 +141,17 @@ class NativePagedAllocator:
     def alloc_extend(self, prefix_lens: torch.Tensor, prefix_lens_cpu: torch.Tensor, seq_lens: torch.Tensor,
                      seq_lens_cpu: torch.Tensor, last_loc: torch.Tensor, extend_num_tokens: int):
         ps = self.page_size
-        pre = prefix_lens_cpu.to(torch.int64)
-        seq = seq_lens_cpu.to(torch.int64)
-        new_pages = int(((seq + ps - 1) // ps - (pre + ps - 1) // ps).sum())
+        bs = int(prefix_lens_cpu.numel())
+        if bs <= 64 and prefix_lens_cpu.shape == seq_lens_cpu.shape:
+            # (a handful of lengths: Python integers cost less than the tensor ops)
+            new_pages = sum((int(s) + ps - 1) // ps - (int(p) + ps - 1) // ps
+                            for p, s in zip(prefix_lens_cpu.reshape(-1).tolist(), seq_lens_cpu.reshape(-1).tolist()))
+        else:
+            pre = prefix_lens_cpu.to(torch.int64)
+            seq = seq_lens_cpu.to(torch.int64)
+            new_pages = int(((seq + ps - 1) // ps - (pre + ps - 1) // ps).sum())
         if new_pages > self.num_pages - self._head:
             return None
-        bs = int(pre.numel())
         out = torch.empty(int(extend_num_tokens), dtype=torch.int64, device=self.device)
         p_dev = prefix_lens.to(device=self.device, dtype=torch.int64).contiguous()
         s_dev = seq_lens.to(device=self.device, dtype=torch.int64).contiguous()

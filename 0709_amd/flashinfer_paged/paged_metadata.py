@@ -16,6 +16,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 from typing import Sequence
 
+import numpy as np
 import torch
 
 from .. import _lib
@@ -51,6 +52,16 @@ class FlashInferPagedKVMetadata:
         non-contiguous page (reads one int32 from the device)."""
         if self.layout_flag is not None and not bool(self.layout_flag.item()):
             raise RuntimeError(LAYOUT_MESSAGE)
+
+
+def _adjacent(slot_paths: Sequence[torch.Tensor], lens: Sequence[int]) -> bool:
+    """The int64 paths follow each other in memory (the pieces of one split slot tensor)."""
+    at = slot_paths[0].data_ptr()
+    for path, n in zip(slot_paths, lens):
+        if path.dtype != torch.int64 or path.data_ptr() != at or (n > 1 and path.stride(0) != 1):
+            return False
+        at += 8 * n
+    return True
 
 
 def build_flashinfer_paged_kv_metadata(
@@ -92,17 +103,22 @@ def build_flashinfer_paged_kv_metadata(
         page_offsets.append(page_offsets[-1] + c)
     last = [n - (c - 1) * ps for n, c in zip(lens, counts)]
     batch = len(lens)
-    # One upload carries offsets, indptr, last-page lengths and sequence
-    # lengths; the int32 outputs are views of one device buffer.
-    host = torch.tensor(path_offsets + page_offsets, dtype=torch.int64)
-    small = torch.tensor(page_offsets + last + lens + [1], dtype=torch.int32)
-    dev64 = host.to(device, non_blocking=True)
-    dev32 = small.to(device, non_blocking=True)
+    # One upload from the pinned ring carries offsets (int64), then indptr,
+    # last-page lengths, sequence lengths and the flag (int32); the int32 outputs
+    # are views of it.
+    wide = np.asarray(path_offsets + page_offsets, dtype=np.int64)
+    small = np.asarray(page_offsets + last + lens + [1], dtype=np.int32)
+    staged = _lib.staging().upload(np.concatenate((wide.view(np.uint8), small.view(np.uint8))), device)
+    dev64 = staged[: wide.nbytes].view(torch.int64)
+    dev32 = staged[wide.nbytes :].view(torch.int32)
     kv_indptr = dev32[: batch + 1]
     kv_last = dev32[batch + 1 : 2 * batch + 1]
     seq_lens = dev32[2 * batch + 1 : 3 * batch + 1]
     flag = dev32[3 * batch + 1 : 3 * batch + 2]
-    slots = torch.cat([p.to(torch.int64) for p in slot_paths]) if batch > 1 else first.to(torch.int64).contiguous()
+    if _adjacent(slot_paths, lens):
+        slots = first  # the paths already lie one behind the other
+    else:
+        slots = torch.cat([p.to(torch.int64) for p in slot_paths]) if batch > 1 else first.to(torch.int64).contiguous()
     total_pages = page_offsets[-1]
     pages = torch.empty(total_pages, dtype=torch.int32, device=device)
     lib = _lib.load()

@@ -179,10 +179,13 @@ def append_token_pool(
     if layer_tables is None:
         layer_tables = _layer_tables(k_layers, v_layers)
     k_tab, v_tab, geom = layer_tables
-    src_stride = k_src[0].stride(0) * k_src[0].element_size()
-    # each distinct source tensor is checked once (callers often pass one
-    # tensor for several layers)
-    for t in {id(t): t for t in (*k_src, *v_src)}.values():
+    first = k_src[0]
+    src_stride = first.stride(0) * first.element_size()
+    dtype, shape, strides = first.dtype, first.shape, first.stride()
+    for t in (*k_src, *v_src):
+        # a source laid out like the first one passes with it
+        if t is not first and t.dtype == dtype and t.shape == shape and t.stride() == strides:
+            continue
         if t.dtype != k_layers[0].dtype:
             raise TypeError(f"source dtype {t.dtype} does not match the pool dtype {k_layers[0].dtype}")
         if int(t.shape[0]) < n or not rows_contiguous(t):
@@ -193,8 +196,8 @@ def append_token_pool(
     lib = _lib.load()
     rc = lib.atlas_kv_append(
         k_tab, v_tab, len(k_layers), *geom.as_head_args(),
-        _lib.ptr_array([int(t.data_ptr()) for t in k_src]),
-        _lib.ptr_array([int(t.data_ptr()) for t in v_src]),
+        _lib.ptr_array(list(map(torch.Tensor.data_ptr, k_src))),
+        _lib.ptr_array(list(map(torch.Tensor.data_ptr, v_src))),
         src_stride, _lib.ptr(dst), 0, n, _lib.stream_of(device),
     )
     _lib.check(rc, "atlas_kv_append")

@@ -415,3 +415,66 @@ def test_paged_metadata_flags_any_bad_slot(dev, ps):
         with pytest.raises(RuntimeError, match="page-aligned"):
             md.assert_layout_valid()
     pm.build_flashinfer_paged_kv_metadata([torch.tensor(good, device=dev)], page_size=ps, sync_check=True)
+
+
+@pytest.mark.parametrize("form", ["split", "gap", "int32", "strided", "reordered", "single"])
+def test_paged_metadata_paths_adjacent_and_apart(dev, form):
+    """Paths that are the pieces of one slot tensor are read in place; every other form is gathered first."""
+    pm = pkg("flashinfer_paged.paged_metadata")
+    ps, lens = 4, [1, 9, 4, 7]
+    paths = [_slot_path([10 * i + j for j in range(1, 4)], n, ps) for i, n in enumerate(lens)]
+    flat = torch.tensor([s for p in paths for s in p], device=dev)
+    if form == "split":
+        got = list(flat.split(lens))
+    elif form == "gap":
+        got = [torch.tensor([0] + p, device=dev)[1:] for p in paths]
+    elif form == "int32":
+        got = list(flat.to(torch.int32).split(lens))
+    elif form == "strided":
+        got = [torch.tensor([x for s in p for x in (s, -1)], device=dev)[::2] for p in paths]
+    elif form == "reordered":
+        got = list(flat.split(lens))[::-1]
+        paths = paths[::-1]
+    else:
+        got, paths = [torch.tensor([x for s in paths[1] for x in (s, -1)], device=dev)[::2]], [paths[1]]
+    md = pm.build_flashinfer_paged_kv_metadata(got, page_size=ps, sync_check=True)
+    exp = ref.paged_metadata(paths, ps)
+    assert md.kv_page_indices.tolist() == exp.kv_page_indices and md.kv_indptr.tolist() == exp.kv_indptr
+    assert md.kv_last_page_len.tolist() == exp.kv_last_page_len and md.seq_lens.tolist() == exp.seq_lens
+
+
+def test_alloc_extend_host_count_matches_for_few_and_many_requests(dev):
+    """The host's page count (Python integers up to 64 requests, tensors beyond) moves the free list's head alike, and
+    refuses an allocation that does not fit."""
+    np_ = pkg("flashinfer_paged.native_pool")
+    for bs in (1, 64, 65):
+        seq = torch.arange(bs) * 7 + 1
+        pre = torch.arange(bs) * 3
+        pages = int(((seq + 15) // 16 - (pre + 15) // 16).sum())
+        for spare, fits in ((0, True), (-1, pages == 0)):
+            if pages + spare <= 0:
+                continue
+            alloc = np_.NativePagedAllocator(size=(pages + spare) * 16, page_size=16, dtype=torch.float16, device=dev)
+            out = alloc.alloc_extend(pre.to(dev), pre, seq.to(dev), seq, pre.to(dev) - 1, int((seq - pre).sum()))
+            assert (out is not None) == fits
+            assert alloc.available_size() == (0 if fits else (pages + spare) * 16)
+
+
+def test_append_token_pool_checks_every_source(dev):
+    """A source unlike the first one is checked by itself: type, rows and row stride."""
+    kv = pkg("kv_ops")
+    pool = [torch.zeros((32, 2, 8), dtype=torch.float16, device=dev) for _ in range(4)]
+    rows = torch.ones((4, 3, 2, 8), dtype=torch.float16, device=dev)
+    dst = torch.tensor([1, 5, 9], device=dev)
+    wide = torch.ones((3, 3, 8), dtype=torch.float16, device=dev)[:, :2]
+    with pytest.raises(TypeError):
+        kv.append_token_pool(pool[:2], pool[2:], [rows[0], rows[1].float()], [rows[2], rows[3]], dst)
+    with pytest.raises(ValueError):
+        kv.append_token_pool(pool[:2], pool[2:], [rows[0], rows[1]], [rows[2], rows[3][:2]], dst)
+    with pytest.raises(ValueError):
+        kv.append_token_pool(pool[:2], pool[2:], [rows[0], rows[1]], [rows[2], wide], dst)
+    with pytest.raises(ValueError):
+        kv.append_token_pool(pool[:2], pool[2:], [rows[0].transpose(1, 2)[..., :2]] * 2, [rows[2], rows[3]], dst)
+    kv.append_token_pool(pool[:2], pool[2:], [rows[0], rows[0]], [rows[2], torch.ones((5, 2, 8), dtype=torch.float16,
+                                                                                    device=dev)], dst)
+    assert all(float(t.float().sum()) == 48.0 for t in pool)
