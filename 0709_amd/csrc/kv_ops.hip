@@ -38,19 +38,19 @@ __global__ __launch_bounds__(kThreads) void kv_move_kernel(LayerTable lt, SlotGe
   *reinterpret_cast<uint4*>(base + dof) = *reinterpret_cast<const uint4*>(base + so);
 }
 
-// One wave per moved slot, for rows of CPR 1 KiB chunks (1 KiB and 2 KiB
-// token rows).  The slot pair is wave-uniform and resolved to byte offsets
-// once; the wave then copies the slot's K and V rows in every layer of the
-// table, LB layers (2 * LB * CPR chunks per lane) in flight.  No branch splits
-// a batch (a branch makes the compiler wait for every outstanding access,
-// stores included, before each store): layers past the last one copy the last
-// layer again, the same bytes to the same place.  dst and src slots are
-// disjoint, so the copies of different waves never overlap.  The stores
-// carry the non-temporal hint (the copies are not read again in this launch;
-// 30.7 -> 24.1 us for a cold 94.6 MB copy-on-write); the loads do not, since
-// a tail page's rows are the source of several copies and hit in L2.
-template <int CPR, int LB>
-__global__ __launch_bounds__(kThreads) void kv_move_rows_kernel(LayerTable lt, SlotGeom g, int num_layers,
+// One wave per moved slot and layer, for rows of CPR 1 KiB chunks (1 KiB and
+// 2 KiB token rows).  The slot pair and the layer are wave-uniform; the wave
+// copies the slot's K and V rows, all loads ahead of the stores.  dst and src
+// slots are disjoint, so the copies of different waves never overlap.  The
+// stores carry the non-temporal hint (the copies are not read again in this
+// launch; 30.7 -> 24.1 us for a cold 94.6 MB copy-on-write); the loads do not,
+// since a tail page's rows are the source of several copies and hit in L2.
+// Small moves are bound by one wave's chain of round trips, so no wave takes
+// several layers: 3 slots of 16 layers 2.3 us (8 layers per batch and wave: 3.3),
+// 312 slots 5.2 (6.2), 2408 slots 20.8 us (22.0), which is 79 MB of rows written at
+// 3.8 TB/s and as many read, most of them from L2.
+template <int CPR>
+__global__ __launch_bounds__(kThreads) void kv_move_rows_kernel(LayerTable lt, SlotGeom g,
                                                                 const int64_t* __restrict__ dst,
                                                                 const int64_t* __restrict__ src, int64_t n) {
   const int64_t item = int64_t(blockIdx.x) * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -58,30 +58,18 @@ __global__ __launch_bounds__(kThreads) void kv_move_rows_kernel(LayerTable lt, S
   const int lane = threadIdx.x & 63;
   const int64_t so = slot_offset(src[item], g) + int64_t(lane) * 16;
   const int64_t dof = slot_offset(dst[item], g) + int64_t(lane) * 16;
-  for (int l0 = 0; l0 < num_layers; l0 += LB) {
-    u32x4v buf[LB][2][CPR];
+  char* kb = const_cast<char*>(lt.k[blockIdx.y]);
+  char* vb = const_cast<char*>(lt.v[blockIdx.y]);
+  u32x4v buf[2][CPR];
 #pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int l = min(l0 + i, num_layers - 1);
-      const char* kb = lt.k[l];
-      const char* vb = lt.v[l];
+  for (int c = 0; c < CPR; ++c) {
+    buf[0][c] = *reinterpret_cast<const u32x4v*>(kb + so + c * 1024);
+    buf[1][c] = *reinterpret_cast<const u32x4v*>(vb + so + c * 1024);
+  }
 #pragma unroll
-      for (int c = 0; c < CPR; ++c) {
-        buf[i][0][c] = *reinterpret_cast<const u32x4v*>(kb + so + c * 1024);
-        buf[i][1][c] = *reinterpret_cast<const u32x4v*>(vb + so + c * 1024);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int l = min(l0 + i, num_layers - 1);
-      char* kb = const_cast<char*>(lt.k[l]);
-      char* vb = const_cast<char*>(lt.v[l]);
-#pragma unroll
-      for (int c = 0; c < CPR; ++c) {
-        __builtin_nontemporal_store(buf[i][0][c], reinterpret_cast<u32x4v*>(kb + dof + c * 1024));
-        __builtin_nontemporal_store(buf[i][1][c], reinterpret_cast<u32x4v*>(vb + dof + c * 1024));
-      }
-    }
+  for (int c = 0; c < CPR; ++c) {
+    __builtin_nontemporal_store(buf[0][c], reinterpret_cast<u32x4v*>(kb + dof + c * 1024));
+    __builtin_nontemporal_store(buf[1][c], reinterpret_cast<u32x4v*>(vb + dof + c * 1024));
   }
 }
 
@@ -311,14 +299,14 @@ extern "C" int atlas_kv_move_slots(const void* const* k_layers, const void* cons
     LayerTable lt;
     fill_table(lt, k_layers, v_layers, l0, nl);
     if (g.row_vecs == 64 || g.row_vecs == 128) {
-      // 1 KiB or 2 KiB token rows: one wave per slot, all layers
-      const dim3 grid(static_cast<unsigned>((n + kThreads / 64 - 1) / (kThreads / 64)));
+      // 1 KiB or 2 KiB token rows: one wave per slot and layer
+      const dim3 grid(static_cast<unsigned>((n + kThreads / 64 - 1) / (kThreads / 64)), static_cast<unsigned>(nl));
       if (g.row_vecs == 64)
-        hipLaunchKernelGGL((kv_move_rows_kernel<1, 8>), grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                           lt, g, nl, dst_slots_dev, src_slots_dev, n);
+        hipLaunchKernelGGL((kv_move_rows_kernel<1>), grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream), lt, g,
+                           dst_slots_dev, src_slots_dev, n);
       else
-        hipLaunchKernelGGL((kv_move_rows_kernel<2, 4>), grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                           lt, g, nl, dst_slots_dev, src_slots_dev, n);
+        hipLaunchKernelGGL((kv_move_rows_kernel<2>), grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream), lt, g,
+                           dst_slots_dev, src_slots_dev, n);
       if ((rc = launch_status("kv_move_rows_kernel"))) return rc;
       continue;
     }
