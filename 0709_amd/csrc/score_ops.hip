@@ -246,23 +246,24 @@ using namespace atlas;
 
 namespace atlas {
 namespace {
-// Chunks per row: about ATLAS_GATHER_TARGET_WGS (row, chunk) workgroups in
-// all, chunks of at least kMinChunk logits (two full batches), at most 256
-// chunks per row.  A workgroup costs its reduction and its arrival, so one per
-// CU is enough: 416 rows x 128256 bf16 logits in one chunk each take 23.8 us
-// (4.5 TB/s), in two 27.5 and in five 25.8; 35 rows in eight chunks 8.3 us, in
-// sixteen 10.1.  (Each workgroup with an L2 write-back at its end, and every
-// lane reading its gather's token in every row: 42.4 and 9.5 us.)
-constexpr int64_t kMinChunk = 16384;
+// Chunks per row: at least about 400 (row, chunk) workgroups in all, 512 for
+// fp32 logits, chunks of at least kMinChunk logits (two full batches), at most
+// 256 chunks per row.  Fewer workgroups leave too few loads in flight, more of
+// them cost their reduction and arrival: rows x 128256 logits in chunks per row
+//   416 bf16: 1 chunk 24.2 us (4.4 TB/s), 2 27.3, 3 26.2 (42.3 with an L2
+//             write-back per workgroup and every lane reading its gather's token
+//             in every row);
+//   200 bf16: 2 17.3, 3 15.6, 6 16.2;      160 fp32: 2 27.0, 4 20.5, 7 20.6;
+//   300 fp32: 1 49.4, 2 32.9, 4 34.2;      500 fp32: 1 54.2, 2 51.2, 3 52.2;
+//   35 rows:  8 chunks of 16384 8.3, sixteen of 8192 10.1.
 struct GatherGeom {
   int num_chunks;
   int64_t chunk_len;
 };
-#ifndef ATLAS_GATHER_TARGET_WGS
-#define ATLAS_GATHER_TARGET_WGS 256
-#endif
-GatherGeom gather_geom(int64_t num_rows, int64_t vocab) {
-  const int64_t want = (ATLAS_GATHER_TARGET_WGS + num_rows - 1) / num_rows;
+constexpr int64_t kMinChunk = 16384;
+GatherGeom gather_geom(int64_t num_rows, int64_t vocab, int esize) {
+  const int64_t workgroups = esize == 4 ? 512 : 400;
+  const int64_t want = (workgroups + num_rows - 1) / num_rows;
   const int64_t by_len = (vocab + kMinChunk - 1) / kMinChunk;
   int64_t chunks = std::max<int64_t>(1, std::min<int64_t>({want, by_len, 256}));
   int64_t len = (vocab + chunks - 1) / chunks;
@@ -275,9 +276,9 @@ GatherGeom gather_geom(int64_t num_rows, int64_t vocab) {
 
 extern "C" int64_t atlas_gather_logprobs_workspace_bytes(int64_t num_rows, int64_t vocab) {
   if (num_rows <= 0 || vocab <= 0 || num_rows >= (int64_t(1) << 31)) return -1;
-  const GatherGeom g = gather_geom(num_rows, vocab);
-  // the slots, then one arrival counter per row
-  return int64_t(size_t(num_rows) * g.num_chunks * sizeof(uint64_t) + size_t(num_rows) * sizeof(uint32_t));
+  const int chunks = std::max(gather_geom(num_rows, vocab, 2).num_chunks, gather_geom(num_rows, vocab, 4).num_chunks);
+  // (of either logit size) the slots, then one arrival counter per row
+  return int64_t(size_t(num_rows) * chunks * sizeof(uint64_t) + size_t(num_rows) * sizeof(uint32_t));
 }
 
 extern "C" int atlas_gather_logprobs(const void* logits_dev, int64_t row_stride, int64_t num_rows,
@@ -299,7 +300,7 @@ extern "C" int atlas_gather_logprobs(const void* logits_dev, int64_t row_stride,
                 "workspace of %lld bytes needed (atlas_gather_logprobs_workspace_bytes), got %zu", (long long)need,
                 workspace_bytes);
   ATLAS_REQUIRE((reinterpret_cast<uintptr_t>(workspace_dev) & 15) == 0, "workspace must be 16-byte aligned");
-  const GatherGeom g = gather_geom(total_rows, vocab);
+  const GatherGeom g = gather_geom(total_rows, vocab, es);
   GatherArgs a{};
   a.logits = static_cast<const char*>(logits_dev);
   a.row_stride_bytes = row_stride * es;
