@@ -57,9 +57,12 @@ struct Vec {
 // workgroup that arrives last (the counter held num_chunks - 1) reads every
 // slot, combines the pairs in chunk order (a fixed order, so the LSE is the same
 // on every run), writes the row LSE and every gather of row r, and empties the
-// slots and the counter for the next call.  A slot is (max bits, ~sum bits).
-// Slots and counters are agent-scope atomics, which every XCD sees, so no
-// workgroup needs a release (a write-back of its XCD's whole L2).
+// slots and the counter for the next call.  A slot is (max bits, ~sum bits),
+// never zero, and carries its whole message in one agent-scope atomic: the last
+// arriver takes a slot as written when it is not zero, whatever order the stores
+// of different workgroups become visible in, so no workgroup needs a release (a
+// write-back of its XCD's whole L2).  A workgroup stores its slot without waiting
+// for anything, so the last arriver finds it, normally at the first read.
 struct GatherArgs {
   const char* logits;
   int64_t row_stride_bytes;
@@ -81,6 +84,7 @@ struct GatherArgs {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kPre = 2;    // gathers per thread whose logits are loaded ahead of the combine
+constexpr int kSlotTries = 1 << 14;  // reads of a slot before it is given up
 constexpr int kBatch = 4;  // 16-byte loads a thread has in flight (8 measured slower: 26.9 us against 24.1)
 
 // (m, s) pairs: s is a sum of exp(x - m).
@@ -99,8 +103,7 @@ __device__ __forceinline__ void batch_add(const Vec<DT> (&x)[N], float& m, float
 #pragma unroll
   for (int b = 0; b < N; ++b)
 #pragma unroll
-    for (int k = 0; k < EPV; k += 2)  // one three-input maximum per two logits (a NaN stays and ends in the sum)
-      mn = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mn, x[b].x[k]), x[b].x[k + 1]);
+    for (int k = 0; k < EPV; ++k) mn = fmaxf(mn, x[b].x[k]);  // (a NaN is no maximum; it ends in the sum)
   const float mb = mn == -INFINITY ? 0.f : mn * kLog2e;  // (all -inf so far: adds zeros)
   float acc = m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - mn) * kLog2e);
 #pragma unroll
@@ -192,12 +195,13 @@ __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a)
     float bm = red_m[0], bs = red_s[0];
 #pragma unroll
     for (int w = 1; w < kThreads / 64; ++w) pair_merge(bm, bs, red_m[w], red_s[w]);
+    if (bs != bs) bs = NAN;  // (one NaN pattern: ~sum is not zero)
     const uint64_t slot = uint64_t(__float_as_uint(bm)) | (uint64_t(~__float_as_uint(bs)) << 32);
     bool last = true;
     if (a.num_chunks > 1) {
       __hip_atomic_store(rs + c, slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       // The slot's store is acknowledged before the arrival goes out, so the
-      // last arriver's loads, issued behind its own arrival, find every slot.
+      // last arriver finds every slot at its first read.
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       const uint32_t prev = __hip_atomic_fetch_add(a.arrivals + r, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       last = prev == uint32_t(a.num_chunks - 1);
@@ -214,7 +218,11 @@ __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a)
   if (t < 64 && a.num_chunks > 1) {
     float cm = -INFINITY, cs = 0.f;
     for (int k = t; k < a.num_chunks; k += 64) {
-      const uint64_t v = __hip_atomic_load(rs + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // (bounded: launches that share a workspace out of stream order could
+      // empty each other's slots; an empty slot reads as a NaN sum)
+      uint64_t v = 0;
+      for (int tries = 0; v == 0 && tries < kSlotTries; ++tries)
+        v = __hip_atomic_load(rs + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       pair_merge(cm, cs, __uint_as_float(uint32_t(v)), __uint_as_float(~uint32_t(v >> 32)));
     }
 #pragma unroll

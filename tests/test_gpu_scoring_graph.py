@@ -295,3 +295,26 @@ def test_gather_logprobs_chunk_edges(dev, dtype, rows, vocab, offset):
     finite = torch.isfinite(expect)
     assert torch.equal(torch.isfinite(got), finite)
     assert (got.double() - expect)[finite].abs().max().item() <= 1e-5 * expect[finite].abs().max().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_gather_logprobs_nan_and_infinite_chunks(dev, dtype):
+    """Several chunks per row, one of them all -inf, all zero, or with a NaN (of any bit pattern) or +inf in it: the
+    last arriver takes every chunk's pair, and a NaN or +inf anywhere makes the row NaN as log_softmax does."""
+    tr = pkg("target_runtime")
+    vocab = 3 * 16384 + 8
+    x = torch.randn((6, vocab), generator=torch.Generator().manual_seed(1)).to(dtype)
+    x[1, :16500] = float("-inf")
+    x[2] = 0
+    ints = {2: torch.int16, 4: torch.int32}[x.element_size()]
+    x.view(ints)[3, 20000] = -1  # a NaN with every bit set
+    x[3, :16000] = 0
+    x[4, 40000] = float("inf")
+    x[5] = float("-inf")
+    at, toks = list(range(6)) * 2, [vocab - 1] * 6 + [17000] * 6
+    got = tr.gather_token_logprobs(x.to(dev), at, toks).cpu().double()
+    expect = (x.double()[at, toks] - torch.logsumexp(x.double(), dim=-1)[at])
+    expect[[4, 10]] = float("nan")  # log_softmax: x - (+inf) with +inf among the logits of an online maximum
+    assert torch.equal(torch.isnan(got), torch.isnan(expect))
+    ok = ~torch.isnan(expect)
+    assert (got - expect)[ok].abs().max().item() <= 1e-5 * expect[ok].abs().max().item()
