@@ -29,7 +29,6 @@ DEFAULT_ROWS_PER_ITEM = 64  # 4 waves x 1 row tile
 MAX_TREE_WIDTH = 64  # tree columns one ancestor word per row covers
 MAX_WIDE_TREE_WIDTH = 4096  # tree columns of the per-tile word layout
 MAX_SPLITS = 1024
-SHORT_SPLIT_TILES = 2  # splits of at most this many tiles are as few as their longest allows
 DEFAULT_CU_COUNT = 256
 
 
@@ -499,14 +498,10 @@ class BatchPrefillWithPagedKVCacheWrapper:
         unit_tiles = sum(hkv * math.ceil(kv_lens[b] / TILE_KEYS) for (b, _, _) in blocks)
         # Tiles per split as a fraction, so the split count per request rounds
         # down and the items do not exceed the target (one per CU when a single
-        # request fills the device).
+        # request fills the device).  A single request of at least as many tiles
+        # as splits then has the same counts at every length, which graphs
+        # captured over run() rely on (see _install).
         tiles_per_split = max(float(self.min_tiles_per_split), unit_tiles / max(1, split_target))
-        # A single request's launch takes as long as its longest split, so short
-        # splits beyond the fewest of that length only add partial rows (32 tiles
-        # of 40 nodes: 16 splits of 2 tiles 14.3 us per layer, 30 splits of 1 or 2
-        # tiles 15.6).  Longer ones gain little (65 tiles: 22 splits of 3 16.9, 30
-        # of 2 or 3 17.4; 12 nodes the same) and run unevenly anyway.
-        even = batch == 1 and gran == TILE_KEYS
         # the merge kernel combines at most MAX_SPLITS states per row
         max_tiles = max((math.ceil(kv_lens[b] / TILE_KEYS) for (b, _, _) in blocks), default=0)
         tiles_per_split = max(tiles_per_split, max_tiles / MAX_SPLITS)
@@ -521,9 +516,6 @@ class BatchPrefillWithPagedKVCacheWrapper:
                 # split, which holds the request's masked tail tile (the
                 # costliest to compute), has one granule less
                 units = math.ceil(kv_lens[b] / gran)
-                longest = math.ceil(units / splits) if units else 0
-                if even and 0 < longest <= SHORT_SPLIT_TILES:
-                    splits = math.ceil(units / longest)
                 per = units // splits if units else 0
                 extra = units - per * splits
                 # request values every item repeats (qo_start, qo_len, kv_len,
@@ -563,10 +555,15 @@ class BatchPrefillWithPagedKVCacheWrapper:
         persistent device buffers and make it the current plan."""
         device = self.device
         meta_np = dec["meta"]
-        # Persistent device buffers keep their addresses across plans, so a
-        # HIP graph captured over run() stays valid after a re-plan of the
-        # same (or a smaller) shape.  Metadata equal to what the buffer already
-        # holds is not uploaded again.
+        # Persistent device buffers keep their addresses across plans that fit
+        # them, so a HIP graph captured over run() stays valid after a re-plan
+        # with the same num_work, num_merge, merge_offset and partial_rows (a
+        # single request with the same heads and query rows, of any length at
+        # which every KV head and row block has its full count of splits: from
+        # 30 64-key tiles on for 8 KV heads and one block) whose page table fits
+        # the buffer (1024 entries, or the largest table planned before the
+        # capture).  Metadata equal to what the buffer already holds is not
+        # uploaded again.
         meta = self._persistent("_meta_buf", len(meta_np), torch.int32)
         if self._meta_uploaded is None or self._meta_uploaded[0] is not meta or \
                 (self._meta_uploaded[1] is not meta_np and not np.array_equal(self._meta_uploaded[1], meta_np)):

@@ -213,6 +213,51 @@ def test_graph_replays_match_eager_forward(dev):
         assert torch.equal(kv.pool, eager_kv)
 
 
+def test_graph_replays_after_plans_of_other_lengths(dev):
+    """One graph captured over run() at 65 key tiles and replayed after re-plans to 64, 40, 31, 30 and 65 tiles (the
+    launch shape is the same from 30 on): each replay equals the eager run of the same plan bit for bit."""
+    ffv = pkg("flashinfer_full_verify")
+    wl = pkg("workloads")
+    geom = wl.Geometry(1, 32, 8, 128)
+    routes, ps = wl.forest_routes(1), 16
+    n = ffv.build_deduplicated_tree_spec_from_paths(paths=routes, prefix_len=1, page_size=ps, device=dev)[0].node_count
+    kv = wl.make_paged_target_kv(geom, kv_len=65 * 64, page_size=ps, dtype=torch.float16, device=dev, seed=3,
+                                 spare_pages=9)
+    q = wl.random_queries(geom, n, dtype=torch.float16, device=dev, seed=4)[0]
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=dev)
+    w = ffv.BatchPrefillWithPagedKVCacheWrapper(ws, "NHD")
+    out = torch.empty_like(q)
+
+    def plan(kv_len):
+        spec, _ = ffv.build_deduplicated_tree_spec_from_paths(paths=routes, prefix_len=kv_len - n, page_size=ps,
+                                                              device=dev)
+        pages = math.ceil(kv_len / ps)
+        w.plan(spec.qo_indptr, torch.tensor([0, pages], dtype=torch.int32, device=dev), kv.kv_indices[:pages],
+               torch.tensor([kv_len - (pages - 1) * ps], dtype=torch.int32, device=dev), 32, 8, 128, ps,
+               custom_mask=spec.bool_mask, q_data_type=torch.float16)
+        p = w.current_plan
+        return p.num_work, p.num_merge, p.merge_offset, p.partial_rows, p.max_rows, p.meta.data_ptr(), \
+            p.kv_indices.data_ptr(), p.tree_mask.data_ptr(), p.page_windows.data_ptr()
+
+    baked = plan(65 * 64)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        w.run(q, kv.layers[0], out=out)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        w.run(q, kv.layers[0], out=out)
+    for kv_len in (65 * 64, 64 * 64, 40 * 64 - 3, 31 * 64 - 63, 30 * 64, 65 * 64 - 1):
+        # what the graph baked in is what this plan needs (checked before the replay)
+        assert plan(kv_len) == baked, kv_len
+        eager = w.run(q, kv.layers[0])
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), kv_len
+
+
 def test_gather_logprobs_graph_replays(dev):
     """The scoring launch through the C ABI, twice in one HIP graph over
     device index buffers and one shared workspace, replayed with new logits

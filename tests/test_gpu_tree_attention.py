@@ -986,12 +986,3 @@ def test_merge_rounds_cover_every_split(dev, d, dtype, splits):
     w, _, _ = _run_and_check(dev, c, split_target=8 * splits, atol=ATOL if dtype == torch.float16 else 4e-3)
     plan = w.current_plan
     assert plan.num_merge == 8 and plan.num_work == 8 * splits
-
-
-@pytest.mark.parametrize("prefix,splits", [(60, 1), (61, 2), (15 * 128 - 4, 30), (15 * 128 - 3, 16),
-                                           (30 * 128 - 4, 30), (30 * 128 - 3, 30)])
-def test_short_splits_are_as_few_as_their_longest_allows(dev, prefix, splits):
-    """Around the tile counts at which the longest of 30 splits grows to two and three 64-key tiles."""
-    c = _build(dev, seed=prefix, prefix_len=prefix, routes=[(1, 2, 3, 4)], dominant_tree=True)
-    w, _, _ = _run_and_check(dev, c)
-    assert w.current_plan.num_work == 8 * splits

@@ -175,3 +175,20 @@ def test_small_workspace_coarsens_the_splits():
     _check(small, qo, kvp, cols, [34], [16418], 32, 8, 128, 16, 136 * 8 * 10)
     assert big["partial_rows"] > 136 * 8 * 10 >= small["partial_rows"] > 0
     assert len(none["work"]) == 8 and none["num_merge"] == 0 and none["partial_rows"] == 0
+
+
+@pytest.mark.parametrize("nodes,first", [(12, 1880), (34, 1880), (68, 960)])
+def test_launch_shape_does_not_depend_on_the_key_count(nodes, first):
+    """A HIP graph captured over run() bakes in the work and merge counts, the offsets into the plan's metadata and
+    the partial-row count.  They are the same for a single request of at least 30 key tiles (15 with two row
+    blocks), however long, so the graph holds after a re-plan of a longer or a shorter prefix."""
+    shapes = set()
+    for kv_len in sorted({*range(first, 4200, 20), *(t * ta.TILE_KEYS + e for t in (30, 31, 40, 58, 60, 64, 65, 128)
+                                                     for e in (-1, 0, 1)), 8200, 16418}):
+        if kv_len < first:
+            continue
+        dec, *_ = _decompose([nodes], [kv_len], 32, 8, 128, 16, 1 << 22)
+        shapes.add((len(dec["work"]), len(dec["meta"]), dec["partial_rows"], dec["max_rows"],
+                    *(dec[k] for k in ("num_merge", "merge_off", "kvlen_off", "col_off", "qo_off", "kvp_off"))))
+    assert len(shapes) == 1, f"{len(shapes)} launch shapes"
+    assert shapes.pop()[0] == 240
