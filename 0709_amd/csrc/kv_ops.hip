@@ -21,7 +21,8 @@ struct InlineItems {
 };
 
 // K[dst] <- K[src], V[dst] <- V[src] for every layer of the table, one vector
-// per thread.
+// per thread.  Pairs with a negative destination (padding) are skipped: the
+// store would land before the layer's first byte.
 __global__ __launch_bounds__(kThreads) void kv_move_kernel(LayerTable lt, SlotGeom g,
                                                            const int64_t* __restrict__ dst,
                                                            const int64_t* __restrict__ src,
@@ -33,9 +34,11 @@ __global__ __launch_bounds__(kThreads) void kv_move_kernel(LayerTable lt, SlotGe
   int64_t item;
   int vec;
   split_row(idx, g, item, vec);
-  const int64_t so = slot_offset(src[item], g) + vec_offset(vec, g);
-  const int64_t dof = slot_offset(dst[item], g) + vec_offset(vec, g);
-  *reinterpret_cast<uint4*>(base + dof) = *reinterpret_cast<const uint4*>(base + so);
+  int64_t from = src[item], to = dst[item];
+  asm volatile("" : "+v"(from), "+v"(to));  // (both loads ahead of the branch)
+  if (to < 0) return;
+  *reinterpret_cast<uint4*>(base + slot_offset(to, g) + vec_offset(vec, g)) =
+      *reinterpret_cast<const uint4*>(base + slot_offset(from, g) + vec_offset(vec, g));
 }
 
 // One wave per moved slot and layer, for rows of CPR 1 KiB chunks (1 KiB and
@@ -78,14 +81,16 @@ struct SrcTable {
   const char* v[ATLAS_MAX_LAYERS_PER_LAUNCH];
 };
 
-// Dense rows -> slots, every layer.  UNROLL vectors per thread, branch-free:
-// vectors past the last one copy the last vector again (the same bytes to the
-// same place), so a thread's slot load and row loads are in flight together.
-// Small appends are bound by that chain of round trips, large ones by HBM.
-// (With a branch around each of four vectors the compiler waits for every
+// Dense rows -> slots, every layer.  UNROLL vectors per thread, loaded without
+// branches: vectors past the last one copy the last vector again (the same
+// bytes to the same place), so a thread's slot load and row loads are in flight
+// together.  Small appends are bound by that chain of round trips, large ones by
+// HBM.  (With a branch around each of four vectors the compiler waits for every
 // vector's loads before it issues the next one's: 200 rows of one layer took
 // 7.8 us and take 2.1, 72 rows of 16 layers 13.8 and 3.0.)  STREAM: loads and
 // stores carry the non-temporal hint, see kStreamBytes.
+// Rows with a negative slot (padding) are skipped: their store would land
+// before the layer's first byte.  All loads stay ahead of these branches.
 template <int UNROLL, bool STREAM>
 __global__ __launch_bounds__(kThreads) void kv_append_kernel(LayerTable lt, SrcTable st, SlotGeom g,
                                                              int64_t src_token_stride,
@@ -114,9 +119,16 @@ __global__ __launch_bounds__(kThreads) void kv_append_kernel(LayerTable lt, SrcT
     const u32x4v* p = reinterpret_cast<const u32x4v*>(sbase + item[u] * src_token_stride + int64_t(vec[u]) * 16);
     buf[u] = STREAM ? __builtin_nontemporal_load(p) : *p;
   }
+  int64_t off[UNROLL];
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) off[u] = slot_offset(slot[u], g) + vec_offset(vec[u], g);
+  // (neither the loads nor the offsets are sunk into the branches below)
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) asm volatile("" : "+v"(buf[u]), "+v"(off[u]));
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u) {
-    u32x4v* p = reinterpret_cast<u32x4v*>(base + slot_offset(slot[u], g) + vec_offset(vec[u], g));
+    if (slot[u] < 0) continue;
+    u32x4v* p = reinterpret_cast<u32x4v*>(base + off[u]);
     if (STREAM) __builtin_nontemporal_store(buf[u], p);
     else *p = buf[u];
   }

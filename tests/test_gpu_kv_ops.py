@@ -481,3 +481,64 @@ def test_move_slots_general_rows(dev, n, dim):
         expect.append(e)
     kv.move_slots(k, v, dst.to(dev), src.to(dev))
     assert all(torch.equal(t.cpu(), e) for t, e in zip(k + v, expect))
+
+
+def _with_room(gen, layers, rows, dev, dim):
+    """K and V layers of ``rows`` [4, dim] token rows, each inside a larger allocation: rows before and behind it."""
+    big = torch.randint(-2 ** 15, 2 ** 15, (2, layers, rows + 128, 4, dim), generator=gen, device=dev,
+                        dtype=torch.int16)
+    return big, [[big[i, l, 64:64 + rows].view(torch.float16) for l in range(layers)] for i in range(2)]
+
+
+@pytest.mark.parametrize("n,layers,dim", [(1, 2, 64), (40, 3, 64), (40, 64, 1024)])
+def test_append_skips_negative_slots(dev, n, layers, dim):
+    """A padding slot (-1, or further below) appends nothing: the rows in front of the layer and every row that is not
+    listed keep their bytes, the other rows arrive (40 rows of 8 KiB, K and V of 64 layers: the streamed form)."""
+    kv = pkg("kv_ops")
+    gen = torch.Generator(device=dev).manual_seed(n)
+    big, (k, v) = _with_room(gen, layers, 64, dev, dim)
+    src = torch.randint(-2 ** 15, 2 ** 15, (2, layers, n, 4, dim), generator=gen, device=dev, dtype=torch.int16)
+    dst = torch.randperm(64, generator=gen, device=dev)[:n].cpu()
+    dst[n // 2] = -1
+    dst[n - 1] = -1 - n
+    expect = big.clone()
+    keep = dst >= 0
+    expect[:, :, 64 + dst[keep].to(dev)] = src[:, :, keep.to(dev)]
+    kv.append_token_pool(k, v, *(list(s.view(torch.float16)) for s in src), dst.to(dev))
+    assert torch.equal(big, expect)
+
+
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+def test_append_paged_skips_negative_slots(dev, layout):
+    """The same for paged layers of 16-token pages, in front of page 0."""
+    kv = pkg("kv_ops")
+    gen = torch.Generator().manual_seed(3)
+    shape = (12, 2, 16, 4, 64) if layout == "NHD" else (12, 2, 4, 16, 64)
+    big = torch.randint(-2 ** 15, 2 ** 15, shape, generator=gen, dtype=torch.int16).to(dev)
+    src = torch.randint(-2 ** 15, 2 ** 15, (2, 20, 4, 64), generator=gen, dtype=torch.int16).to(dev)
+    dst = torch.randperm(128, generator=gen)[:20]
+    dst[[0, 9, 19]] = torch.tensor([-1, -16, -17])
+    expect = big.clone()
+    for i, slot in enumerate(dst.tolist()):
+        for part in range(2):
+            if slot >= 0:
+                page = expect[2 + slot // 16, part]
+                (page if layout == "NHD" else page.transpose(0, 1))[slot % 16] = src[part, i]
+    layer = big[2:10].view(torch.float16)
+    kv.append_paged([layer], *([s.view(torch.float16)] for s in src), dst_slots=dst.to(dev), kv_layout=layout)
+    assert torch.equal(big, expect)
+
+
+def test_move_slots_general_rows_skip_negative_destinations(dev):
+    """A pair with a padding destination moves nothing (rows that are not 1 or 2 KiB)."""
+    kv = pkg("kv_ops")
+    gen = torch.Generator(device=dev).manual_seed(5)
+    big, (k, v) = _with_room(gen, 3, 64, dev, 40)
+    perm = torch.randperm(64, generator=gen, device=dev).cpu()
+    src, dst = perm[:24], perm[24:48].clone()
+    dst[[0, 11, 23]] = torch.tensor([-1, -2, -24])
+    expect = big.clone()
+    keep = dst >= 0
+    expect[:, :, 64 + dst[keep].to(dev)] = big[:, :, 64 + src[keep].to(dev)]
+    kv.move_slots(k, v, dst.to(dev), src.to(dev))
+    assert torch.equal(big, expect)
