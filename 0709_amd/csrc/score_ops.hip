@@ -87,11 +87,16 @@ constexpr int kPre = 2;    // gathers per thread whose logits are loaded ahead o
 constexpr int kSlotTries = 1 << 14;  // reads of a slot before it is given up
 constexpr int kBatch = 4;  // 16-byte loads a thread has in flight (8 measured slower: 26.9 us against 24.1)
 
-// (m, s) pairs: s is a sum of exp(x - m).
+// (m, s) pairs: s is a sum of exp(x - m), and while m is -inf 0, or NaN when a
+// NaN has been met: a maximum drops a NaN, so the sum carries it.  exp_ref is
+// what exponents are taken relative to: with it, -inf adds 0 and keeps a NaN,
+// without a branch.
+__device__ __forceinline__ float exp_ref(float m) { return m == -INFINITY ? 0.f : m; }
+
 __device__ __forceinline__ void pair_merge(float& m, float& s, float m2, float s2) {
   const float mn = fmaxf(m, m2);
-  if (mn == -INFINITY) return;
-  s = s * __builtin_amdgcn_exp2f((m - mn) * kLog2e) + s2 * __builtin_amdgcn_exp2f((m2 - mn) * kLog2e);
+  const float ref = exp_ref(mn);
+  s = s * __builtin_amdgcn_exp2f((m - ref) * kLog2e) + s2 * __builtin_amdgcn_exp2f((m2 - ref) * kLog2e);
   m = mn;
 }
 
@@ -103,9 +108,10 @@ __device__ __forceinline__ void batch_add(const Vec<DT> (&x)[N], float& m, float
 #pragma unroll
   for (int b = 0; b < N; ++b)
 #pragma unroll
-    for (int k = 0; k < EPV; ++k) mn = fmaxf(mn, x[b].x[k]);  // (a NaN is no maximum; it ends in the sum)
-  const float mb = mn == -INFINITY ? 0.f : mn * kLog2e;  // (all -inf so far: adds zeros)
-  float acc = m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - mn) * kLog2e);
+    for (int k = 0; k < EPV; ++k) mn = fmaxf(mn, x[b].x[k]);
+  const float ref = exp_ref(mn);
+  const float mb = ref * kLog2e;
+  float acc = s * __builtin_amdgcn_exp2f((m - ref) * kLog2e);
 #pragma unroll
   for (int b = 0; b < N; ++b) {
     float part = 0.f;

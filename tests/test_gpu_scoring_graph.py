@@ -363,3 +363,41 @@ def test_gather_logprobs_nan_and_infinite_chunks(dev, dtype):
     assert torch.equal(torch.isnan(got), torch.isnan(expect))
     ok = ~torch.isnan(expect)
     assert (got - expect)[ok].abs().max().item() <= 1e-5 * expect[ok].abs().max().item()
+
+
+def _row_lse(dev, logits):
+    """Every row's log-sum-exp, from the launch itself (logits: [rows, vocab], any row start)."""
+    lib_mod = pkg("_lib")
+    lib = lib_mod.load()
+    rows, vocab = logits.shape
+    need = int(lib.atlas_gather_logprobs_workspace_bytes(rows, vocab))
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    lse = torch.empty(rows, dtype=torch.float32, device=dev)
+    rc = lib.atlas_gather_logprobs(lib_mod.ptr(logits), logits.stride(0), rows, None, 0, 0, vocab,
+                                   lib_mod.dtype_code(logits.dtype), None, None, 0, lib_mod.ptr(lse), None,
+                                   lib_mod.ptr(ws), need, lib_mod.stream_of(dev))
+    lib_mod.check(rc, "atlas_gather_logprobs")
+    return lse.cpu().double()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [5001, 3 * 16384 + 9])
+def test_gather_logprobs_nan_among_minus_infinity(dev, dtype, vocab):
+    """A NaN that only -inf precedes or surrounds makes the row NaN: in a 16-byte load, in a single element before and
+    behind them, as a whole chunk; -inf alone does not.  (Rows start one element past a 16-byte boundary.)"""
+    inf, nan = float("inf"), float("nan")
+    flat = torch.randn(7 * vocab + 1, generator=torch.Generator().manual_seed(vocab)).to(dtype)
+    x = flat[1:].view(7, vocab)
+    x[0, : vocab // 2] = -inf
+    x[0, 1000] = nan          # then -inf up to the middle, then finite
+    x[1] = -inf
+    x[1, 0] = nan             # a single element ahead of the first 16-byte load
+    x[2] = -inf
+    x[2, vocab - 1] = nan     # one behind the last
+    x[3, : vocab // 3] = nan  # a whole chunk (or its first third), the rest finite
+    x[4] = nan
+    x[5, : vocab // 2] = -inf
+    x[6] = -inf
+    got = _row_lse(dev, flat.to(dev)[1:].view(7, vocab))
+    assert torch.isnan(got).tolist() == [True] * 5 + [False] * 2
+    assert abs(float(got[5] - torch.logsumexp(x[5].double(), 0))) <= 1e-5 * abs(float(got[5])) and float(got[6]) == -inf
