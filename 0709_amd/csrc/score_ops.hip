@@ -2,6 +2,7 @@
 // log-probabilities of the verified tokens, so a verify needs one small
 // device-to-host copy instead of one scalar read per token.
 #include <algorithm>
+#include <cfloat>
 
 #include "common.hpp"
 
@@ -83,6 +84,7 @@ struct GatherArgs {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+constexpr float kFar = 2.3e38f;  // kLog2e * kFar is finite
 constexpr int kPre = 2;    // gathers per thread whose logits are loaded ahead of the combine
 constexpr int kSlotTries = 1 << 14;  // reads of a slot before it is given up
 constexpr int kBatch = 4;  // 16-byte loads a thread has in flight (8 measured slower: 26.9 us against 24.1)
@@ -110,7 +112,9 @@ __device__ __forceinline__ void batch_add(const Vec<DT> (&x)[N], float& m, float
 #pragma unroll
     for (int k = 0; k < EPV; ++k) mn = fmaxf(mn, x[b].x[k]);
   const float ref = exp_ref(mn);
-  const float mb = ref * kLog2e;
+  // (past kFar the product overflows: kept finite, so the sum is 0 and not NaN
+  // until a larger logit comes, and folded again at the end if none does)
+  const float mb = DT == ATLAS_DTYPE_F16 ? ref * kLog2e : __builtin_amdgcn_fmed3f(ref * kLog2e, -FLT_MAX, FLT_MAX);
   float acc = s * __builtin_amdgcn_exp2f((m - ref) * kLog2e);
 #pragma unroll
   for (int b = 0; b < N; ++b) {
@@ -170,6 +174,18 @@ __global__ __launch_bounds__(kThreads) void gather_logprobs_kernel(GatherArgs a)
     Vec<DT> x[1];
     x[0].load(vrow + v * 16);
     batch_add<DT, 1>(x, m, s);
+  }
+  // Nothing but logits masked with the type's lowest value (or a maximum as
+  // large): the same vectors again, by difference.
+  if (DT != ATLAS_DTYPE_F16 && __builtin_fabsf(m) > kFar && m != -INFINITY) {
+    s = 0.f;
+#pragma unroll 1
+    for (v = t; v < nv; v += kThreads) {
+      Vec<DT> x;
+      x.load(vrow + v * 16);
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) s += __builtin_amdgcn_exp2f((x.x[k] - m) * kLog2e);
+    }
   }
   const int singles = static_cast<int>((a0 - c0) + (c1 - a1));
   if (t < singles) {

@@ -401,3 +401,29 @@ def test_gather_logprobs_nan_among_minus_infinity(dev, dtype, vocab):
     got = _row_lse(dev, flat.to(dev)[1:].view(7, vocab))
     assert torch.isnan(got).tolist() == [True] * 5 + [False] * 2
     assert abs(float(got[5] - torch.logsumexp(x[5].double(), 0))) <= 1e-5 * abs(float(got[5])) and float(got[6]) == -inf
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [5000, 5001, 3 * 16384 + 8, 3 * 16384 + 9])
+def test_gather_logprobs_rows_masked_with_the_lowest_value(dev, dtype, vocab):
+    """Logits masked with the type's lowest value count as nothing beside others, wherever the run of them lies; a row
+    of nothing else has it as its log-sum-exp.  log2(e) times it overflows fp32 for bf16 and fp32 logits.  (Rows
+    that start on a 16-byte boundary and rows that do not; fp32 sums: 1e-5.)"""
+    lo = torch.finfo(dtype).min
+    off = vocab % 2
+    flat = torch.randn(6 * vocab + 1, generator=torch.Generator().manual_seed(vocab)).to(dtype)
+    x = flat[off: off + 6 * vocab].view(6, vocab)
+    x[0, : vocab // 2] = lo
+    x[1, vocab // 2:] = lo
+    x[2, : vocab - 1] = lo
+    x[3] = lo
+    x[4, ::2] = lo
+    x[5, : vocab // 3] = lo
+    x[5, vocab // 3: vocab // 2] = float("-inf")
+    dx = flat.to(dev)[off: off + 6 * vocab].view(6, vocab)
+    got = _row_lse(dev, dx)
+    expect = torch.logsumexp(x.double(), dim=1)
+    assert ((got - expect).abs() <= 1e-5 * expect.abs().clamp_min(1)).all()
+    lp = pkg("target_runtime").gather_token_logprobs(dx, [0, 2, 4], [vocab - 1] * 3).cpu().double()
+    want = x.double()[[0, 2, 4], vocab - 1] - expect[[0, 2, 4]]
+    assert ((lp - want).abs() <= 1e-5 * want.abs().clamp_min(1)).all()
