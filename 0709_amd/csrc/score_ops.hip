@@ -52,9 +52,9 @@ struct Vec {
 
 // Workgroup (c, r) reads chunk c of logits row r once: the chunk's maximum m
 // and the sum of exp(x - m), kept online per thread over batches of kBatch
-// 16-byte loads, then reduced over the
-// workgroup.  It stores the pair into its slot of the row, waits until the
-// store is acknowledged and counts itself in on the row's arrival counter; the
+// 16-byte loads, then reduced over the workgroup.  It stores the pair into its
+// slot of the row, waits until the store is acknowledged and counts itself in on
+// the row's arrival counter (a row of one chunk needs neither); the
 // workgroup that arrives last (the counter held num_chunks - 1) reads every
 // slot, combines the pairs in chunk order (a fixed order, so the LSE is the same
 // on every run), writes the row LSE and every gather of row r, and empties the
@@ -63,7 +63,10 @@ struct Vec {
 // arriver takes a slot as written when it is not zero, whatever order the stores
 // of different workgroups become visible in, so no workgroup needs a release (a
 // write-back of its XCD's whole L2).  A workgroup stores its slot without waiting
-// for anything, so the last arriver finds it, normally at the first read.
+// for anything, so the last arriver finds it, normally at the first read; a slot
+// still zero after kSlotTries reads counts as a NaN sum.  Only launches in stream
+// order may share a workspace: another launch's pair in a slot is taken as this
+// launch's own.
 struct GatherArgs {
   const char* logits;
   int64_t row_stride_bytes;
@@ -276,30 +279,53 @@ using namespace atlas;
 
 namespace atlas {
 namespace {
-// Chunks per row: at least about 400 (row, chunk) workgroups in all, 512 for
-// fp32 logits, chunks of at least kMinChunk logits (two full batches), at most
-// 256 chunks per row.  Fewer workgroups leave too few loads in flight, more of
-// them cost their reduction and arrival: rows x 128256 logits in chunks per row
-//   416 bf16: 1 chunk 24.2 us (4.4 TB/s), 2 27.3, 3 26.2 (42.3 with an L2
-//             write-back per workgroup and every lane reading its gather's token
-//             in every row);
-//   200 bf16: 2 17.3, 3 15.6, 6 16.2;      160 fp32: 2 27.0, 4 20.5, 7 20.6;
-//   300 fp32: 1 49.4, 2 32.9, 4 34.2;      500 fp32: 1 54.2, 2 51.2, 3 52.2;
-//   35 rows:  8 chunks of 16384 8.3, sixteen of 8192 10.1.
+// Chunks per row, from the row count and the vocabulary in batches (what a
+// workgroup folds in one round: kBatch 16-byte loads per thread, 8192 16-bit or
+// 4096 fp32 logits).  A launch takes as long as one workgroup's rounds in series,
+// 0.4 to 0.5 us each, plus 1.3 to 1.8 us for slots and arrivals when a row has
+// more than one chunk, until rows x chunks fills the device; beyond that each
+// further workgroup costs its reduction and its arrival.  So: chunks of few
+// batches for few rows, and of more batches the more workgroups there are
+// already.  The limits on rows x chunks lie where the next length is faster;
+// more than 12 arrivals on one row's counter only pay in small launches; rows of
+// up to 4 batches, and 16-bit rows from the stated count on, are faster as
+// one chunk.  A chunk is whole batches (what is left of one is folded a vector at a
+// time, each a round trip of its own), or the row's even share where that leaves
+// half a batch or less.
+//
+// Measured, us (graph replays over cold logits): this rule against chunks of at
+// least 16384 logits for 400 or 512 workgroups, and one chunk per row:
+//   x 128256 bf16     1 row  4.8,  6.1, 12.7     5  5.6,  6.8, 13.4    20  7.2,  7.9, 13.8
+//                       50   8.5,  9.6, 18.0   100 10.1, 11.3, 18.4   170 13.2, 13.3, 19.5
+//                      200  15.4, 16.9, 19.9   300 20.9, 21.6, 22.2   399 24.1, 27.3, 24.0
+//                      416  24.4, 24.5, 24.4   (a write-back of L2 per workgroup and
+//                      every lane reading its gather's token in every row: 41.4)
+//   x 128256 fp32     1      5.0,  7.0, 23.7     5  6.3,  8.1, 26.0    20  7.6,  9.2, 26.9
+//                       50  10.8, 12.2, 37.4   100 14.1, 14.4, 38.2   200 23.4, 24.1, 41.4
+//                      399  42.1, 42.1, 49.3   512 51.1, 53.2, 53.3
+//   x 32001 bf16      1      4.8,  5.7,  4.7    35  6.5,  7.1,  6.5   200  9.1, 10.0,  9.1
+//   x 32001 fp32      1      4.6,  5.9,  5.5    35  6.7,  8.4,  9.5   200 11.2, 12.8, 14.1
+// Over 1 to 600 rows of 9001 to 152064 logits the rule is within 6 % of the best
+// chunk length tried, mostly within 2 %.
 struct GatherGeom {
   int num_chunks;
   int64_t chunk_len;
 };
-constexpr int64_t kMinChunk = 16384;
 GatherGeom gather_geom(int64_t num_rows, int64_t vocab, int esize) {
-  const int64_t workgroups = esize == 4 ? 512 : 400;
-  const int64_t want = (workgroups + num_rows - 1) / num_rows;
-  const int64_t by_len = (vocab + kMinChunk - 1) / kMinChunk;
-  int64_t chunks = std::max<int64_t>(1, std::min<int64_t>({want, by_len, 256}));
-  int64_t len = (vocab + chunks - 1) / chunks;
-  len = (len + 7) / 8 * 8;
-  chunks = (vocab + len - 1) / len;
-  return GatherGeom{int(chunks), len};
+  const int64_t batch = int64_t(kBatch) * kThreads * (16 / esize);
+  const int64_t batches = (vocab + batch - 1) / batch;
+  if (batches <= 4 || (esize == 2 && num_rows >= std::max<int64_t>(224, 24 * batches)))
+    return GatherGeom{1, (vocab + 7) / 8 * 8};
+  const int64_t most16[] = {128, 400, 600, 500, 768}, most32[] = {128, 400, 600, 1024, 1024};
+  int64_t per = 1, chunks = batches;
+  while (chunks > 1) {
+    const int64_t i = std::min<int64_t>(per, 5) - 1;
+    if (num_rows * chunks <= (chunks > 12 ? 150 : esize == 4 ? most32[i] : most16[i])) break;
+    per = (batches + chunks - 2) / (chunks - 1);  // the next length with fewer chunks
+    chunks = (batches + per - 1) / per;
+  }
+  const int64_t even = (vocab + chunks * 8 - 1) / (chunks * 8) * 8;  // (chunks start on 8 logits)
+  return GatherGeom{int(chunks), even % batch <= batch / 2 ? even : per * batch};
 }
 }  // namespace
 }  // namespace atlas

@@ -427,3 +427,19 @@ def test_gather_logprobs_rows_masked_with_the_lowest_value(dev, dtype, vocab):
     lp = pkg("target_runtime").gather_token_logprobs(dx, [0, 2, 4], [vocab - 1] * 3).cpu().double()
     want = x.double()[[0, 2, 4], vocab - 1] - expect[[0, 2, 4]]
     assert ((lp - want).abs() <= 1e-5 * want.abs().clamp_min(1)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,vocab", [(1, 32769), (2, 40961), (25, 40961), (26, 40961), (80, 40961), (81, 40961),
+                                        (223, 40001), (224, 40001), (13, 50257), (150, 50257), (1, 151 * 4096 + 1)])
+def test_gather_logprobs_chunk_rule(dev, dtype, rows, vocab):
+    """Both sides of the chunk rule's lines (16-bit rows turn to one chunk at 224, chunks grow from one batch to two and
+    more with the rows), last chunks of a single logit, even shares, and more than 150 batches, against float64."""
+    tr = pkg("target_runtime")
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    logits = torch.randn((rows, vocab), generator=gen, device=dev).mul_(3).to(dtype)
+    at = [r for r in range(rows) for _ in range(2)]
+    toks = [t for r in range(rows) for t in (vocab - 1, (r * 7919) % vocab)]
+    got = tr.gather_token_logprobs(logits, at, toks).double()
+    expect = torch.cat([x.double() - torch.logsumexp(x.double(), -1, keepdim=True) for x in logits.split(32)])[at, toks]
+    assert (got - expect).abs().max().item() <= 1e-5 * expect.abs().max().item()
