@@ -235,22 +235,23 @@ __global__ __launch_bounds__(kSweepThreads) void prune_paths_gather_kernel(
   gather_values(g, out, threadIdx.x, kSweepThreads);
 }
 
-// Page tables from concatenated slot paths.  `lanes` lanes (a power of two, at
-// most 64) per page: the page id is the slot of the page's first token divided
-// by page_size; the layout check requires that first slot to be page-aligned
-// and every later slot of the page (within the path length) to follow it
+// Page tables from concatenated slot paths.  1 << lane_shift lanes (at most 64)
+// per page: the page id is the slot of the page's first token divided by
+// page_size; the layout check requires that first slot to be page-aligned and
+// every later slot of the page (within the path length) to follow it
 // contiguously, each lane checking every lanes-th slot of its page.
 // Bound by latency: a page's slots are one round of coalesced loads (8 prompts
 // of 4.8k tokens in all, pages of 64: 4.3 us; with one thread walking a page's slots,
 // each load behind the last one's compare, 12.3 us).
 __global__ __launch_bounds__(256) void paged_metadata_kernel(const int64_t* slots, const int64_t* path_offsets,
                                                              const int64_t* page_offsets, int num_paths,
-                                                             int64_t total_pages, int64_t page_size, int lanes,
+                                                             int64_t total_pages, int64_t page_size, int lane_shift,
                                                              int validate, int32_t* page_indices,
                                                              int32_t* layout_ok) {
+  const int lanes = 1 << lane_shift;
   const int sub = threadIdx.x & (lanes - 1);
-  const int per_block = 256 / lanes;
-  for (int64_t pg = int64_t(blockIdx.x) * per_block + int(threadIdx.x) / lanes; pg < total_pages;
+  const int per_block = 256 >> lane_shift;
+  for (int64_t pg = int64_t(blockIdx.x) * per_block + (threadIdx.x >> lane_shift); pg < total_pages;
        pg += int64_t(gridDim.x) * per_block) {
     // Binary search for the path owning this page.
     int lo = 0, hi = num_paths - 1;
@@ -267,7 +268,7 @@ __global__ __launch_bounds__(256) void paged_metadata_kernel(const int64_t* slot
           static_cast<int32_t>(first >= 0 ? first / page_size : -((-first + page_size - 1) / page_size));
     if (validate) {
       bool ok = sub != 0 || (((first % page_size) + page_size) % page_size) == 0;
-      for (int64_t i = begin + sub; i < end; i += lanes) ok &= slots[i] == first + (i - begin);
+      for (int64_t i = begin + (sub != 0 ? sub : lanes); i < end; i += lanes) ok &= slots[i] == first + (i - begin);
       if (!ok) *layout_ok = 0;
     }
   }
@@ -680,12 +681,12 @@ extern "C" int atlas_paged_metadata(const int64_t* slots_dev, const int64_t* pat
   ATLAS_REQUIRE(!validate || layout_ok_dev, "validation needs a layout flag");
   if (total_pages <= 0) return ATLAS_OK;
   // enough lanes for a page's slots in one round; one lane when they are not read
-  int lanes = 1;
-  while (validate && lanes < 64 && lanes < page_size) lanes *= 2;
-  const int64_t per_block = 256 / lanes;
+  int lane_shift = 0;
+  while (validate && lane_shift < 6 && (int64_t(1) << lane_shift) < page_size) ++lane_shift;
+  const int64_t per_block = 256 >> lane_shift;
   const int blocks = static_cast<int>(std::min<int64_t>((total_pages + per_block - 1) / per_block, 2048));
   hipLaunchKernelGGL(paged_metadata_kernel, dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     slots_dev, path_offsets_dev, page_offsets_dev, num_paths, total_pages, page_size, lanes,
+                     slots_dev, path_offsets_dev, page_offsets_dev, num_paths, total_pages, page_size, lane_shift,
                      validate, kv_page_indices_dev, layout_ok_dev);
   return launch_status("paged_metadata_kernel");
 }
