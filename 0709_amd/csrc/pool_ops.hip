@@ -709,8 +709,11 @@ extern "C" int atlas_alloc_extend_slots(const int64_t* prefix_lens_dev, const in
   if (bs == 0) return ATLAS_OK;
   ATLAS_REQUIRE(prefix_lens_dev && seq_lens_dev && last_loc_dev && free_pages_dev && out_dev, "NULL buffer");
   // The token counts are on the device: a few requests get up to 16 workgroups
-  // each (4096 tokens in one round), many requests share 512 workgroups.
-  const int across = std::min(bs, 512);
+  // each (4096 tokens in one round); beyond 1024 requests a workgroup takes several
+  // in turn (requests of one or two tokens: 700 4.1 us, 1024 4.7, 4096 13.1; with 512
+  // workgroups 4.7, 5.3 and 15.0, with 2048 4.1, 4.7 and 16.3, since every workgroup
+  // reads the requests before its own; one thread per request 4.4, 5.1 and 14.1).
+  const int across = std::min(bs, 1024);
   const int along = std::max(1, std::min(16, 512 / across));
   hipLaunchKernelGGL(alloc_extend_kernel, dim3(across, along), dim3(kExtendThreads), 0,
                      static_cast<hipStream_t>(stream), prefix_lens_dev, seq_lens_dev, last_loc_dev, free_pages_dev,

@@ -378,10 +378,11 @@ def test_gather_i64_segments(dev, target):
 
 
 @pytest.mark.parametrize("ps,seqs", [(16, [1]), (64, [5000]), (1, [3, 700]), (16, [257, 256, 255, 1, 4097]),
-                                     (7, [20] * 600), (64, [63, 64, 65] * 30)])
+                                     (7, [20] * 600), (64, [63, 64, 65] * 30), (7, [3] * 1023), (7, [2, 9] * 513),
+                                     (16, [1] * 2100)])
 def test_alloc_extend_many_tokens_per_request(dev, ps, seqs):
     """Requests of more tokens than one workgroup, or one round of them, takes (256 and 4096), more requests than
-    the grid is wide (512), and page remainders, against the oracle allocator; every other request starts inside
+    the grid is wide (1024), and page remainders, against the oracle allocator; every other request starts inside
     a page, and request 0 appends nothing when there is a second one."""
     lib = _lib()
     rng = np.random.default_rng(len(seqs) + ps)
