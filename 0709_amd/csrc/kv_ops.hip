@@ -322,9 +322,14 @@ extern "C" int atlas_kv_move_slots(const void* const* k_layers, const void* cons
       if ((rc = launch_status("kv_move_rows_kernel"))) return rc;
       continue;
     }
-    hipLaunchKernelGGL(kv_move_kernel, copy_grid(n, g, nl, 1), dim3(kThreads), 0,
-                       static_cast<hipStream_t>(stream), lt, g, dst_slots_dev, src_slots_dev, n);
-    if ((rc = launch_status("kv_move_kernel"))) return rc;
+    // (a grid holds fewer than 2^32 threads, one per vector here)
+    const int64_t most = (int64_t(1) << 31) / g.row_vecs;
+    for (int64_t i0 = 0; i0 < n; i0 += most) {
+      const int64_t m = std::min(most, n - i0);
+      hipLaunchKernelGGL(kv_move_kernel, copy_grid(m, g, nl, 1), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+                         lt, g, dst_slots_dev + i0, src_slots_dev + i0, m);
+      if ((rc = launch_status("kv_move_kernel"))) return rc;
+    }
   }
   return ATLAS_OK;
 }

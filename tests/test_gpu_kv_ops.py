@@ -542,3 +542,16 @@ def test_move_slots_general_rows_skip_negative_destinations(dev):
     expect[:, :, 64 + dst[keep].to(dev)] = big[:, :, 64 + src[keep].to(dev)]
     kv.move_slots(k, v, dst.to(dev), src.to(dev))
     assert torch.equal(big, expect)
+
+
+def test_move_slots_of_more_vectors_than_a_grid_holds(dev):
+    """65537 slots of 1 MiB rows are more than 2^32 16-byte vectors: several launches.  (Every copy but the last one
+    takes row 0 to row 1, so the pool stays small.)"""
+    kv = pkg("kv_ops")
+    k, v = (torch.randint(-2 ** 15, 2 ** 15, (4, 8, 2 ** 16), device=dev, dtype=torch.int16) for _ in range(2))
+    src = torch.zeros(2 ** 16 + 1, dtype=torch.int64, device=dev)
+    dst = src + 1
+    src[-1], dst[-1] = 2, 3
+    expect = [t[[0, 0, 2, 2]].clone() for t in (k, v)]
+    kv.move_slots([k.view(torch.float16)], [v.view(torch.float16)], dst, src)
+    assert torch.equal(k, expect[0]) and torch.equal(v, expect[1])
