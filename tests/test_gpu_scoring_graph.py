@@ -31,8 +31,9 @@ def test_gather_logprobs_matches_oracle(dev, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape,offset", [((7, 1003), 0), ((5, 1001), 1), ((3, 9), 1)])
 def test_gather_logprobs_unaligned_and_ragged_rows(dev, dtype, shape, offset):
-    """Row starts that are not 16-byte aligned (scalar path) and vocabularies
-    that are not a multiple of the vector width (vector path tail)."""
+    """Row starts that are not 16-byte aligned (single elements ahead of the
+    first 16-byte load) and vocabularies that are not a multiple of the vector
+    width (single elements behind the last)."""
     tr = pkg("target_runtime")
     gen = torch.Generator().manual_seed(shape[1] + offset)
     full = (torch.randn((shape[0], shape[1] + offset), generator=gen) * 4).to(dtype)
